@@ -82,6 +82,12 @@ def lib() -> ctypes.CDLL:
         handle.gptq2d_sweep_fused_kron_f32.argtypes = [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I32,
                                                        _P, _P, _F64, _F64, _I32, _P, _P, _I64, _I64, _I64, _P]
         handle.gptq2d_sweep_fused_kron_f32.restype = ctypes.c_int
+        handle.gptq2d_sweep_split_f32.argtypes = [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I32,
+                                                  _AP, _AP, _AP, _I32, _P, _AP, _P, _AP, _F64, _F64, _I32, _P, _P, _I64,
+                                                  _I64, _I64, _P, _I64, _P]
+        handle.gptq2d_sweep_split_f32.restype = ctypes.c_int
+        handle.gptq2d_sweep_split_workspace.argtypes = [_I64, _I64, _I32, _AP, _AP, _AP]
+        handle.gptq2d_sweep_split_workspace.restype = ctypes.c_int64
         handle.gptq2d_viterbi_workspace.argtypes = [_I64, _I64, _I32, _I32, _I32]
         handle.gptq2d_viterbi_workspace.restype = ctypes.c_int64
         handle.gptq2d_int_code_bits.argtypes = [_F64, _F64]

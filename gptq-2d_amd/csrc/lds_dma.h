@@ -74,6 +74,21 @@ __device__ __forceinline__ void dma_load_so(__amdgpu_buffer_rsrc_t r, float* dst
         : "v"(off), "s"(r), "s"(lds), "s"(soff)
         : "memory");
 }
+// Three consecutive 1 KB LDS-direct loads (128 bits per lane each): bytes [off + 1024 p, off + 1024 p + 16) past
+// the scalar offset `soff` of buffer r go to dst + 1024 p + 16 lane, p = 0..2.  The instruction offset counts in
+// the memory address and in the LDS address alike, and in the range check (soff does not), so one M0 serves
+// the three and an `off` past the extent writes zeros.
+__device__ __forceinline__ void dma_load_3k(__amdgpu_buffer_rsrc_t r, void* dst, int off, int soff) {
+  const unsigned lds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(lds_float*)dst);
+  unsigned saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %4 offen lds\n\t"
+      "buffer_load_dwordx4 %1, %2, %4 offen offset:1024 lds\n\tbuffer_load_dwordx4 %1, %2, %4 offen offset:2048 "
+      "lds\n\ts_mov_b32 m0, %0"
+      : "=&s"(saved)
+      : "v"(off), "s"(r), "s"(lds), "s"(soff)
+      : "memory");
+}
 // All of this wave's LDS-direct loads have landed.
 __device__ __forceinline__ void wait_dma() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 

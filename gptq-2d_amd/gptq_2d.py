@@ -211,6 +211,35 @@ def _fused_spec(quantizer, quantizer_inputs, y, batch_shape, rows=False):
     return None
 
 
+# Largest workspace of the split-operand sweep (an fp32 sweep that would need more runs on fp32 operands)
+SPLIT_WORKSPACE_MAX = 32 << 30
+
+
+def _run_split(y, l, u, m, n, batch_shape, spec, outer_block_size, p, q):
+    """The fused fp32 sweep on split operands (gptq2d_sweep_split_f32); False where it does not apply."""
+    if y.dtype != torch.float32 or m >= 1 << 20 or n >= 1 << 20 or batch_shape.numel() > 65535:
+        return False
+    kron = isinstance(u, KroneckerU)
+    bshape, nd = _hip.i64_array(batch_shape), len(batch_shape)
+    lstr = _hip.batch_strides(l, batch_shape)
+    ustr = _hip.i64_array([0] * nd) if kron else _hip.batch_strides(u, batch_shape)
+    need = _hip.lib().gptq2d_sweep_split_workspace(m, n, nd, bshape, lstr, ustr)
+    if not 0 <= need <= SPLIT_WORKSPACE_MAX:
+        return False
+    c, e = torch.empty_like(y), torch.empty_like(y)
+    work = torch.empty(max(need, 16), dtype=torch.uint8, device=y.device)
+    qa, qb = spec["qa"], spec["qb"]
+    up, uq = (u.outer, u.inner) if kron else (None, None)
+    _hip.call_untyped(
+        "sweep_split_f32", _hip.ptr(y), _hip.ptr(c), _hip.ptr(e), _hip.ptr(l), None if kron else _hip.ptr(u),
+        _hip.ptr(up), _hip.ptr(uq), up.size(0) if kron else 0, uq.size(0) if kron else 0, m, n, p, q, nd, bshape, lstr,
+        ustr, spec["kind"], _hip.ptr(qa), _hip.batch_strides(qa, batch_shape) if qa is not None else None, _hip.ptr(qb),
+        _hip.batch_strides(qb, batch_shape) if qb is not None else None, spec["qmin"], spec["qmax"],
+        spec.get("dtype16", 0), _hip.ptr(spec["ypre"]), _hip.ptr(spec.get("sout")), _outer_tiles(outer_block_size), 0,
+        -1, _hip.ptr(work), work.numel(), _hip.stream(y.device))
+    return True
+
+
 def _run_fused_kron(y, l, u, m, n, spec, outer_block_size, p=1, q=1):
     """The fused sweep of one matrix with U given by its Kronecker factors (gptq2d_sweep_fused_kron_f32)."""
     c = torch.empty_like(y)  # zeroed by the library
@@ -328,7 +357,9 @@ def _sweep(x, l, u, quantizer, super_entry_shape, inner_block_size, outer_block_
     if kron and not _kron_fusable(y, l, u, batch_shape, spec):
         u, kron = u.dense(), False
     with torch.cuda.device(x.device):
-        if kron:
+        if spec is not None and _run_split(y, l, u, m, n, batch_shape, spec, outer_block_size, p, q):
+            pass
+        elif kron:
             _run_fused_kron(y, l, u, m, n, spec, outer_block_size, p, q)
         elif spec is not None:
             _run_fused(y, l, u, m, n, batch_shape, spec, outer_block_size, p, q)

@@ -231,6 +231,26 @@ int gptq2d_sweep_fused_kron_f32(float* y, float* c, float* e, const float* l, co
                                 float* ypre, float* scale_out, int64_t outer_tiles, int64_t stage_begin,
                                 int64_t stage_end, void* stream);
 
+/* gptq2d_sweep_fused_se_f32 / gptq2d_sweep_fused_kron_f32 (U = up (x) uq where up is not NULL; no batch then) with
+ * the products between tiles formed on the bf16 matrix cores from operands split into three bf16 pieces each (x =
+ * h + m + l; six exact piece products per product, fp32 accumulation: sums at least as close to 64 bits as
+ * those of the fp32 instruction, and sums that are not finite formed again in fp32).  work: 16-byte aligned device
+ * workspace of gptq2d_sweep_split_workspace bytes, overwritten; stage_begin > 0 resumes with the c of the call
+ * before.  Any row length and alignment; m, n < 2^20, nq % 16 == 0; arguments are checked before any device work
+ * (the same reference counterparts as gptq2d_sweep_fused_se). */
+int gptq2d_sweep_split_f32(float* y, float* c, float* e, const float* l, const float* u, const float* up,
+                           const float* uq, int64_t np, int64_t nq, int64_t m, int64_t n, int64_t p, int64_t q,
+                           int32_t bnd, const int64_t* bshape, const int64_t* lstride, const int64_t* ustride,
+                           int32_t qkind, const float* qa, const int64_t* qa_stride, const float* qb,
+                           const int64_t* qb_stride, double qmin, double qmax, int32_t dtype16, float* ypre,
+                           float* scale_out, int64_t outer_tiles, int64_t stage_begin, int64_t stage_end, void* work,
+                           int64_t work_bytes, void* stream);
+
+/* Workspace bytes of gptq2d_sweep_split_f32 (-1 for sizes it does not take): the split E and C of every matrix, and
+ * of L and U one copy where the batch shares them (all batch strides 0).  No counterpart in the reference. */
+int64_t gptq2d_sweep_split_workspace(int64_t m, int64_t n, int32_t bnd, const int64_t* bshape, const int64_t* lstride,
+                                     const int64_t* ustride);
+
 /* Largest B m n (elements per matrix of the batch) gptq2d_sweep_fused_noalloc_* accepts for elements of
  * elem_bytes bytes (4 or 8; -1 otherwise): 2^24 for float, 2^23 for double.  No counterpart in the
  * reference (see gptq2d_sweep_fused_noalloc). */
