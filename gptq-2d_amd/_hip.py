@@ -44,6 +44,7 @@ _SIGNATURES = {
     "absmax_scale": [_P, _P, _I64, _I64, _I64, _I64, _F64, _F64, _I32, _P],
     "absmax_quantize_se": [_P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _F64, _F64, _I32, _P, _P],
     "ldl_of_inverse": [_P, _P, _P, _P, _I64, _I64, _I64, _P],
+    "embed": [_P, _P, _I64, _I64, _I64, _I64, _P],
     "ldl": [_P, _P, _P, _P, _I64, _I64, _I64, _P],
     "ldl_of_inverse_part": [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I32, _P],
     "ldl_of_inverse_pair": [_P, _P, _P, _P, _I64, _I64, _P, _P, _P, _P, _I64, _I64, _I32, _P, _P, _P],

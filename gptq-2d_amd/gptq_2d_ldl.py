@@ -37,6 +37,33 @@ def _side_streams(device: torch.device):
     return _SIDE_STREAMS[key]
 
 
+# Sizes from which, and below which, a matrix whose rows are not on 16-byte boundaries is factored inside an
+# aligned one: 602 fp32 1.15 -> 0.44 ms, 1531 3.20 -> 1.00, 8190 23.5 -> 7.6; fp64 777 0.91 -> 0.70, 4099 5.41 ->
+# 4.04.  Smaller ones keep the library's own sequence, the one its entry points for parts of a factorisation take
+# (301 fp32: 0.48 against 0.29 ms); from PAD_MAX on the two larger copies would be 1 GiB (fp32) and more each.
+PAD_MIN, PAD_MAX = 640, 16384
+
+
+def _pad(m: torch.Tensor, size: int) -> int:
+    """Rows of identity to add to m (a multiple of the block size) so that the kernels that move 16 bytes of a
+    row at a time take it: fp32 the two-level factorisation and the MFMA inverse levels, fp64 the strip's
+    narrow product.  (A batch the embedding's grid cannot number stays as it is.)"""
+    k, align = m.size(-1), 16 // m.element_size()
+    if k % align == 0 or not PAD_MIN <= k < PAD_MAX or m.numel() > 65535 * k * k:
+        return 0
+    pad = size
+    while (k + pad) % align:
+        pad += size
+    return pad
+
+
+def _embed(m: torch.Tensor, kd: int, off: int) -> torch.Tensor:
+    """[batch, k, k] at row and column off of a kd x kd identity; kd < k: its part from -off on."""
+    out = m.new_empty(m.size(0), kd, kd)
+    _hip.call("embed", m.dtype, _hip.ptr(out), _hip.ptr(m), m.size(0), kd, m.size(-1), off, _hip.stream(m.device))
+    return out
+
+
 def _factor(name: str, m: torch.Tensor, size: int, check: bool) -> torch.Tensor:
     assert m.dim() >= 2 and m.size(-1) == m.size(-2), "expected square matrices [..., k, k]"
     assert m.dtype in (torch.float32, torch.float64), "expected float32 or float64"
@@ -47,12 +74,20 @@ def _factor(name: str, m: torch.Tensor, size: int, check: bool) -> torch.Tensor:
     batch = m.shape[:-2]
     src = m.reshape(-1, k, k).contiguous()
     nb = src.size(0)
-    out = torch.empty_like(src)
-    work = torch.empty_like(src)
     info = torch.zeros(nb, dtype=torch.int32, device=m.device)
+    pad = _pad(src, size)
+    # the identity goes where the factorisation comes last: before M for the reversed order of
+    # ldl_of_inverse, after it for ldl, so that info counts the minors of M
+    lead = pad if name == "ldl_of_inverse" else 0
     with torch.cuda.device(m.device):
-        _hip.call(name, m.dtype, _hip.ptr(src), _hip.ptr(out), _hip.ptr(work), _hip.ptr(info), nb, k, size,
+        if pad:
+            src = _embed(src, k + pad, lead)
+        out = torch.empty_like(src)
+        work = torch.empty_like(src)
+        _hip.call(name, m.dtype, _hip.ptr(src), _hip.ptr(out), _hip.ptr(work), _hip.ptr(info), nb, k + pad, size,
                   _hip.stream(m.device))
+        if pad:
+            out = _embed(out, k, -lead)
     if check and nb and k:
         bad = info.cpu()
         if bool((bad != 0).any()):
@@ -105,40 +140,48 @@ def feedback_factors_of_grams(G: torch.Tensor, H: torch.Tensor, super_entry_shap
         k = m.size(-1)
         assert size > 0 and k % size == 0, "the block size must divide the matrix size"
         assert size <= MAX_BLOCK[m.dtype], f"diagonal blocks up to {MAX_BLOCK[m.dtype]} are supported for {m.dtype}"
-        jobs.append((m, size, k))
+        jobs.append((m, size, k, _pad(m, size)))
     out = []
     upper = False  # whether out[1] holds U itself (else the second factor, U its transpose)
     with torch.cuda.device(G.device):
         # each factor's buffers on its stream's pool
         bufs = []
-        for s, (m, size, k) in zip(streams, jobs):
+        for s, (m, size, k, pad) in zip(streams, jobs):
             with torch.cuda.stream(s):
                 src = m.reshape(-1, k, k).contiguous()
+                if pad:
+                    src = _embed(src, k + pad, pad)
                 bufs.append((src, torch.empty_like(src), torch.empty_like(src),
                              torch.zeros(src.size(0), dtype=torch.int32, device=m.device)))
         (sa, oa, wa, ia), (sb, ob, wb, ib) = bufs
-        (_, pa, ka), (_, pb, kb) = jobs
+        (_, pa, ka, da), (_, pb, kb, db) = jobs
         if max(sa.size(0), sb.size(0)) > 1:
             # batches: each factor's matrices in one batched call on its own stream, whose matrices of the
             # fp32 two-level path share every Cholesky launch (up to 16 at a time)
-            for s, (m, size, k), (src, o, w, info) in zip(streams, jobs, bufs):
+            for s, (m, size, k, pad), (src, o, w, info) in zip(streams, jobs, bufs):
                 with torch.cuda.stream(s):
                     _hip.call("ldl_of_inverse", src.dtype, _hip.ptr(src), _hip.ptr(o), _hip.ptr(w), _hip.ptr(info),
-                              src.size(0), k, size, _hip.stream(m.device))
+                              src.size(0), k + pad, size, _hip.stream(m.device))
         elif sa.dtype == sb.dtype and sa.size(0) == sb.size(0):
             # U = ldl_of_inverse(H)^T written by the library (unit diagonal): no transposed copy in the sweep
             upper = pb == 1
             sp = [ctypes.c_void_p(s.cuda_stream) for s in streams]
             for b in range(sa.size(0)):
                 _hip.call("ldl_of_inverse_pair", sa.dtype, _hip.ptr(sa[b]), _hip.ptr(oa[b]), _hip.ptr(wa[b]),
-                          _hip.ptr(ia[b:b + 1]), ka, pa, _hip.ptr(sb[b]), _hip.ptr(ob[b]), _hip.ptr(wb[b]),
-                          _hip.ptr(ib[b:b + 1]), kb, pb, int(upper), *sp)
+                          _hip.ptr(ia[b:b + 1]), ka + da, pa, _hip.ptr(sb[b]), _hip.ptr(ob[b]), _hip.ptr(wb[b]),
+                          _hip.ptr(ib[b:b + 1]), kb + db, pb, int(upper), *sp)
         else:  # one matrix each, of different dtypes: each factor on its own stream
-            for s, (m, size, k), (src, o, w, info) in zip(streams, jobs, bufs):
+            for s, (m, size, k, pad), (src, o, w, info) in zip(streams, jobs, bufs):
                 with torch.cuda.stream(s):
                     for b in range(src.size(0)):
-                        _part(src[b], o[b], w[b], info[b:b + 1], k, size, 0, -1, 1)
-        out = [oa.reshape(G.shape), ob.reshape(H.shape)]
+                        _part(src[b], o[b], w[b], info[b:b + 1], k + pad, size, 0, -1, 1)
+        for f, s in enumerate(streams[:2]):
+            if jobs[f][3]:
+                with torch.cuda.stream(s):  # U' = diag(I, U) as L' = diag(I, L)
+                    out.append(_embed((oa, ob)[f], jobs[f][2], -jobs[f][3]))
+            else:
+                out.append((oa, ob)[f])
+        out = [t.reshape(m.shape) for t, m in zip(out, (G, H))]
     # streams[2]'s work is ordered before the last launches of streams[0] and [1] (events)
     for s, t in zip(streams, out):
         main.wait_stream(s)

@@ -167,6 +167,11 @@ extern "C" {
   /* Unit lower (block) triangular L with M = L Lambda L^T (ldl, gptq_2d_reference.py:52-55). */       \
   int gptq2d_ldl_##SUF(const T* m, T* out, T* work, int* info, int64_t batch, int64_t k, int64_t size,              \
                        void* stream);                                                                               \
+  /* dst [batch, kd, kd] = src [batch, ks, ks] at row and column off of an identity (off >= 0,          \
+   * off + ks <= kd), or the part of src from row and column -off on (off <= 0, kd - off <= ks): a     \
+   * matrix brought to rows on 16-byte boundaries for the factorisations, and its factor taken out.    \
+   * No counterpart in the reference. */                                                              \
+  int gptq2d_embed_##SUF(T* dst, const T* src, int64_t batch, int64_t kd, int64_t ks, int64_t off, void* stream);   \
   /* Strided batched GEMM D = beta D + alpha A B with triangular operand structure (tri: 0 dense,      \
    * 1 lower, 2 upper) -- the building block of the LDL; exported for tests.  No reference            \
    * counterpart (torch.linalg inside the reference's ldl_of_inverse). */                             \

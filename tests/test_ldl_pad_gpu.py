@@ -1,0 +1,105 @@
+"""Factors of matrices whose rows are not on 16-byte boundaries, taken inside an aligned one: diag(I, M) has the
+factor diag(I, L).  Against the fp64 reference computed from the definition, with the error of an aligned factor of
+about the same size as the yardstick."""
+
+import pytest
+import torch
+
+import _hip
+import gptq_2d_ldl as LDL
+import instances
+from oracle import algorithms as A
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _err(got, ref):
+    return ((got.double().cpu() - ref).abs().max() / ref.abs().max()).item()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("kd,ks,off,batch", [(5, 3, 2, 2), (3, 3, 0, 1), (3, 5, -2, 3), (4, 7, 0, 2), (1028, 1027, 1, 1),
+                                             (1027, 1030, -3, 2), (1, 1, 0, 1)])
+def test_embed(kd, ks, off, batch, dtype):
+    src = torch.randn(batch, ks, ks, device=DEV, dtype=dtype)
+    got = LDL._embed(src, kd, off)
+    if kd >= ks:
+        ref = torch.eye(kd, device=DEV, dtype=dtype).repeat(batch, 1, 1)
+        ref[:, off:off + ks, off:off + ks] = src
+    else:
+        ref = src[:, -off:-off + kd, -off:-off + kd]
+    assert got.equal(ref)
+
+
+@pytest.mark.parametrize("kd,ks,off", [(5, 3, 3), (3, 5, -3), (5, 3, -1)])
+def test_embed_refuses_what_does_not_fit(kd, ks, off):
+    with pytest.raises(_hip.GPTQ2DError):
+        LDL._embed(torch.zeros(1, ks, ks, device=DEV), kd, off)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("k,size", [(641, 1), (1531, 1), (2051, 1), (645, 5), (1533, 21), (901, 53), (639, 1)])
+def test_padded_factor(k, size, dtype):
+    m = instances.wishart_factor(k, .5, 11)
+    # both sides solve the same well-conditioned system (alpha .5), so the padded factor's error is that of an
+    # aligned one of the next size up to the draw: within 4 times, and never above k eps
+    other = k + (-k) % (4 * size)
+    ma = instances.wishart_factor(other, .5, 11)
+    for fn, of in ((LDL.ldl_of_inverse, A.ldl_of_inverse), (LDL.ldl, A.ldl)):
+        x = m.to(DEV, dtype)
+        got = fn(x, size)
+        assert got.is_contiguous() and got.shape == (k, k)
+        err = _err(got, of(x.double().cpu(), size))
+        xa = ma.to(DEV, dtype)
+        yard = _err(fn(xa, size), of(xa.double().cpu(), size))
+        eps = torch.finfo(dtype).eps
+        print(f"{fn.__name__} {k} {size} {dtype}: {err:.1e}, aligned {yard:.1e}", flush=True)
+        assert err <= max(4 * yard, 4 * eps) and err < k * eps
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("ka,kb,pa,pb", [(1000, 1531, 1, 1), (777, 645, 7, 5), (1030, 1030, 1, 2)])
+def test_padded_pair_and_batch(ka, kb, pa, pb, dtype):
+    """Pairs and batches equal single calls bit for bit, as for aligned sizes."""
+    a = torch.stack([instances.wishart_factor(ka, .5, s) for s in (1, 2)]).to(DEV, dtype)
+    b = torch.stack([instances.wishart_factor(kb, .5, s) for s in (3, 4)]).to(DEV, dtype)
+    la = [LDL.ldl_of_inverse(x, pa) for x in a]
+    ub = [LDL.ldl_of_inverse(x, pb).t() for x in b]
+    lo, up = LDL.feedback_factors_of_grams(a[0], b[0], (pa, pb))
+    assert lo.equal(la[0]) and up.equal(ub[0])
+    lo, up = LDL.feedback_factors_of_grams(a, b, (pa, pb))
+    assert lo.equal(torch.stack(la)) and up.equal(torch.stack(ub))
+    t = b.transpose(-1, -2)  # other strides, the same values
+    assert LDL.ldl_of_inverse(t, pb).equal(LDL.ldl_of_inverse(t.contiguous(), pb))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("at", [0, 700, 1030])
+def test_padded_failure_names_the_minor(at, dtype):
+    """An indefinite matrix reports the order of its own minor, not of the embedding's."""
+    k = 1031
+    m = torch.eye(k, device=DEV, dtype=dtype)
+    m[at, at] = -1
+    with pytest.raises(torch.linalg.LinAlgError, match=f"order {at + 1} "):
+        LDL.ldl(m)
+    with pytest.raises(torch.linalg.LinAlgError, match=f"order {k - at} "):
+        LDL.ldl_of_inverse(m)
+    with pytest.raises(torch.linalg.LinAlgError, match=f"order {k - at} "):
+        LDL.feedback_factors_of_grams(m, torch.eye(1000, device=DEV, dtype=dtype))
+
+
+def test_padded_under_capture():
+    """check=False: one graph of the padded factorisation, replayed on new values."""
+    k = 1027
+    x = instances.wishart_factor(k, .5, 5).to(DEV).float()
+    LDL.ldl_of_inverse(x, check=False)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = LDL.ldl_of_inverse(x, check=False)
+    for seed in (5, 6, 7):
+        x.copy_(instances.wishart_factor(k, .5, seed).to(DEV).float())
+        graph.replay()
+        torch.cuda.synchronize()
+        assert out.equal(LDL.ldl_of_inverse(x))
