@@ -48,6 +48,7 @@ EXTRA_FLAGS = {
     "gemm.hip": VGPR_MFMA,
     "flush.hip": VGPR_MFMA,
     "ldl.hip": VGPR_MFMA,
+    "trmm_mfma.hip": VGPR_MFMA,
 }
 
 

@@ -39,6 +39,7 @@
 // ldl), which call torch.linalg.cholesky and solve_triangular.
 #include "linalg.h"
 #include "lds_dma.h"
+#include "split_mma.h"
 
 
 #include <array>
@@ -48,7 +49,6 @@
 
 namespace {
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 template <typename T>
 struct LdlBlock;
@@ -807,32 +807,20 @@ __global__ __launch_bounds__(256) void normalize_block_solve_kernel(T* __restric
   }
 }
 
-// Rank-K update of a lower trapezoid on fp32 MFMA (v_mfma_f32_32x32x2_f32):
+// Rank-K update of a lower trapezoid on split operands (split_mma.h):
 //   D -= P P^T  on  D = W[r0.., r0..] (R x R; lower triangle, columns < C),  P = W[r0.., pc .. pc + K)
-// with K a multiple of 32.  One workgroup per 128 x 128 block (bi, bj), four waves of 64 x 64 (2 x 2
-// MFMA blocks each).  The K loop walks k-tiles of 32: both panels of a k-tile (the block's 128 rows
-// of P, and the 128 rows that are its columns) are loaded one k-tile ahead straight into LDS
-// (buffer loads with the LDS destination bit), double-buffered, one barrier per k-tile; rows past R
-// (A) or past min(R, C) (B) load as zeros.  Both panels use the same layout -- P's k runs along a row
-// for both operands of D = P P^T: float f of a panel holds row f / 32 and k = 4 (q ^ quad_swizzle(row))
-// + f % 4, q = (f % 32) / 4 (16-byte k-quads XOR-swizzled by row, lds_dma.h, so that the lanes reading one
-// quad of different rows hit different bank groups), and every fragment read is 128 bits.  Lane l (i = l % 32, h = l / 32)
-// feeds A(i, 16 h + s) and B(16 h + s, i) to MFMA s; the accumulators hold
-// D(8 (r / 4) + 4 h + r % 4, i).  The epilogue subtracts the products from D in place (read all
-// 16 entries of a block, then write), masked to the lower triangle, to i < R and to j < C.
+// with K a multiple of 16.  One workgroup per 128 x 128 block (bi, bj), four waves of 64 x 64.  P's k runs along a
+// row for both operands, so a thread's eight values of a k-tile are two 128-bit loads; rows past R (A) or past
+// min(R, C) (B) load as zeros.  The accumulators hold D(8 (r / 4) + 4 h + r % 4, i) for lane i + 32 h.  The epilogue
+// subtracts the products from D in place (read all 16 entries of a block, then write), masked to the lower
+// triangle, to i < R and to j < C.
 //
 // The same kernel serves the three updates of the two-level Cholesky below: a panel's update of the
 // next panel's columns (C = 64), its update of the rest of its strip (rank 64), and a strip's update of the
 // whole trailing triangle (rank 512 or 1024).
 constexpr int WB = 128;  // block edge
-constexpr int WK = 32;   // k-tile depth
 
-struct WideLds {
-  float a[2][WB * WK];
-  float b[2][WB * WK];
-};
-
-__device__ __forceinline__ void syrk_wide_block(WideLds& sm, float* __restrict__ w, int64_t ld, int64_t r0, int R,
+__device__ __forceinline__ void syrk_wide_block(SplitLds& sm, float* __restrict__ w, int64_t ld, int64_t r0, int R,
                                                 int C, int64_t pc, int K, int bi, int bj) {
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -847,87 +835,16 @@ __device__ __forceinline__ void syrk_wide_block(WideLds& sm, float* __restrict__
       matrix_rsrc(w + (r0 + I0) * ld + pc, arows > 0 ? (int64_t)(arows - 1) * ld + K : 0);
   const __amdgpu_buffer_rsrc_t rpb =
       matrix_rsrc(w + (r0 + J0) * ld + pc, brows > 0 ? (int64_t)(brows - 1) * ld + K : 0);
+  const int row = 32 * wave + li;
+  const int aoff = row < arows ? (row * ild + 8 * hh) * 4 : OOB, boff = row < brows ? (row * ild + 8 * hh) * 4 : OOB;
+  const int aoff1 = row < arows ? aoff + 16 : OOB, boff1 = row < brows ? boff + 16 : OOB;
 
-  // per-lane staging offsets of the wave's four 128-bit loads per panel and k-tile
-  int aoff[4], boff[4];
-#pragma unroll
-  for (int x = 0; x < 4; ++x) {
-    const int f = (wave + 4 * x) * 256 + 4 * lane;
-    const int row = f >> 5, kq = ((f >> 2) & 7) ^ quad_swizzle(row);
-    aoff[x] = row < arows ? (row * ild + 4 * kq) * 4 : OOB;
-    boff[x] = row < brows ? (row * ild + 4 * kq) * 4 : OOB;
-  }
-  // a block whose rows and columns all lie inside the update takes the k offset in the loads' scalar field:
-  // no vector instruction beside the MFMA bursts
-  const bool full = I0 + WB <= R && J0 + WB <= CR;
-  auto issue = [&](int t, int buf) {
-    if (full) {
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        const int f0 = (wave + 4 * x) * 256;
-        dma_load_so<4>(rpa, &sm.a[buf][f0], aoff[x], t * WK * 4);
-        dma_load_so<4>(rpb, &sm.b[buf][f0], boff[x], t * WK * 4);
-      }
-      return;
-    }
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const int f0 = (wave + 4 * x) * 256;
-      dma_load<4>(rpa, &sm.a[buf][f0], aoff[x] == OOB ? OOB : aoff[x] + t * WK * 4);
-      dma_load<4>(rpb, &sm.b[buf][f0], boff[x] == OOB ? OOB : boff[x] + t * WK * 4);
-    }
-  };
-
-  // a wave with nothing to write (above the diagonal, right of C or below R) still loads and waits
   const bool act = !(bi == bj && wy < wx) && J0 + 64 * wx < C && I0 + 64 * wy < R;
   floatx16 acc[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int d = 0; d < 2; ++d)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[a][d][r] = 0.f;
-
-  const int sw = quad_swizzle(li);
-  const int a_base = (64 * wy + li) * WK, b_base = (64 * wx + li) * WK;
-  auto step = [&](int t, auto cur_c) {
-    constexpr int cur = decltype(cur_c)::value;
-    __syncthreads();  // buffer cur is complete; buffer 1 - cur is no longer read
-    if (t + 1 < K / WK) issue(t + 1, 1 - cur);
-    if (act) {
-      const float* as = &sm.a[cur][a_base];
-      const float* bs = &sm.b[cur][b_base];
-      float4 fa[2][2], fb[2][2];
-      auto frag = [&](int v, int slot) {
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-          fa[slot][a] = *reinterpret_cast<const float4*>(as + a * 32 * WK + 4 * ((4 * hh + v) ^ sw));
-          fb[slot][a] = *reinterpret_cast<const float4*>(bs + a * 32 * WK + 4 * ((4 * hh + v) ^ sw));
-        }
-      };
-      frag(0, 0);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        if (v < 3) frag(v + 1, (v + 1) & 1);
-#pragma unroll
-        for (int s2 = 0; s2 < 4; ++s2)
-#pragma unroll
-          for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int d = 0; d < 2; ++d)
-              acc[a][d] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[v & 1][a][s2], fb[v & 1][d][s2], acc[a][d], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    wait_dma();  // this wave's loads of k-tile t + 1 have landed before the next barrier
-  };
-  issue(0, 0);
-  wait_dma();
-  for (int t = 0; t < K / WK; t += 2) {
-    step(t, std::integral_constant<int, 0>{});
-    if (t + 1 < K / WK) step(t + 1, std::integral_constant<int, 1>{});
-  }
-  if (!act) return;
+  split_block_product(
+      sm, 0, K / 16, acc, [&](int t, float (&x)[8]) { load_row8(rpa, aoff, aoff1, 64 * t, x); },
+      [&](int t, float (&x)[8]) { load_row8(rpb, boff, boff1, 64 * t, x); });
+  if (!act) return;  // nothing to write: above the diagonal, right of C or below R
   // the block of D at rows r0 + I0 .., columns r0 + J0 .. (a resource based there: offsets below 128 rows)
   const __amdgpu_buffer_rsrc_t rd = matrix_rsrc(w + (r0 + I0) * ld + r0 + J0, (int64_t)(arows - 1) * ld + WB);
 #pragma unroll
@@ -948,27 +865,35 @@ __device__ __forceinline__ void syrk_wide_block(WideLds& sm, float* __restrict__
     }
 }
 
-// Workgroup lin of n renumbered so that each XCD (own L2) runs a contiguous share of the blocks: the
-// hardware deals workgroup w to XCD w % 8.
-__device__ __forceinline__ int64_t xcd_contiguous(int64_t lin, int64_t n) {
-  const int64_t base = n / 8, extra = n % 8, xcd = lin % 8;
-  return xcd * base + (xcd < extra ? xcd : extra) + lin / 8;
+// Block (bi, bj) number id of a lower trapezoid of nb block rows and nbc block columns, numbered in bands of 8 block
+// rows, column by column inside a band: the blocks that run together on an XCD (64: two on each of its 32 CUs)
+// share 8 row panels and as many column panels, 16 panels from beyond the L2 instead of the 65 of a block row.
+constexpr int BAND = 8;
+__device__ __forceinline__ int64_t trapezoid_before(int64_t row, int64_t nbc) {
+  return row <= nbc ? row * (row + 1) / 2 : nbc * (nbc + 1) / 2 + (row - nbc) * nbc;
 }
-
-// Block (bi, bj) number id of a lower trapezoid of blocks with nbc block columns, numbered row by
-// row: the triangle of the first nbc block rows, then nbc blocks per row.
-__device__ __forceinline__ void trapezoid_block(int64_t id, int64_t nbc, int& bi, int& bj) {
-  const int64_t tri = nbc * (nbc + 1) / 2;
-  if (id >= tri) {
-    bi = (int)(nbc + (id - tri) / nbc);
-    bj = (int)((id - tri) % nbc);
+__device__ __forceinline__ void trapezoid_block(int64_t id, int64_t nb, int64_t nbc, int& bi, int& bj) {
+  int64_t row;  // the block row that holds number id if numbered row by row: the same band
+  if (id >= nbc * (nbc + 1) / 2) {
+    row = nbc + (id - nbc * (nbc + 1) / 2) / nbc;
+  } else {
+    row = (int64_t)((sqrt(8.0 * (double)id + 1.0) - 1.0) * 0.5);
+    while ((row + 1) * (row + 2) / 2 <= id) ++row;
+    while (row * (row + 1) / 2 > id) --row;
+  }
+  const int64_t r0 = row / BAND * BAND, nr = nb - r0 < BAND ? nb - r0 : BAND;
+  int64_t at = id - trapezoid_before(r0, nbc);
+  const int64_t full = r0 + 1 < nbc ? r0 + 1 : nbc;  // columns that have all rows of the band
+  if (at < full * nr) {
+    bi = (int)(r0 + at % nr);
+    bj = (int)(at / nr);
     return;
   }
-  int64_t ti = (int64_t)((sqrt(8.0 * (double)id + 1.0) - 1.0) * 0.5);
-  while ((ti + 1) * (ti + 2) / 2 <= id) ++ti;
-  while (ti * (ti + 1) / 2 > id) --ti;
-  bi = (int)ti;
-  bj = (int)(id - ti * (ti + 1) / 2);
+  at -= full * nr;
+  int64_t c = full;
+  while (at >= nr - (c - r0)) at -= nr - (c - r0), ++c;
+  bi = (int)(c + at);
+  bj = (int)c;
 }
 
 // Workgroups of a trapezoid update (R x R lower triangle, columns < C; C <= R).
@@ -998,7 +923,7 @@ struct PanelGroup {
 template <int PB>
 __global__ __launch_bounds__(256, 2) void syrk_strip_kernel(PanelGroup grp, int64_t ld, int64_t r0, int R,
                                                             int64_t pc, int K, int64_t sc) {
-  __shared__ __align__(16) WideLds sm;
+  __shared__ __align__(16) SplitLds sm;
   const PanelPtrs& p = grp.p[blockIdx.y];
   if (blockIdx.x == gridDim.x - 1) {
     stage_to_w<float, PB>(p.w, ld, sc, PB, p.stage);
@@ -1008,22 +933,27 @@ __global__ __launch_bounds__(256, 2) void syrk_strip_kernel(PanelGroup grp, int6
 }
 
 // Look-ahead step of the fp32 Cholesky: workgroups [0, n_potrf) factor and solve panel j0; the
-// others apply a pending trapezoid update (square W[r0.., r0..], R x R, columns < C, rank K from
-// P = W[r0.., pc .. pc + K)).  The two touch disjoint columns, so the panel's latency-bound
+// others apply a pending trapezoid update.  The two touch disjoint columns, so the panel's latency-bound
 // factorisation runs beside the throughput-bound update.
 // upc >= 0: the panel first takes the rank-PB update of the panel at columns [upc, upc + PB) itself.
 // copy != nullptr: the last workgroup moves that earlier panel's staged diagonal block (at column
 // copy_j0, PB rows) into W.  The matrix: entry blockIdx.y of the group (the copy set in all or none).
+
+// A trapezoid update of n blocks: square W[r0.., r0..] (R x R), columns < C, rank K from P = W[r0.., pc .. pc + K).
+struct Update {
+  int64_t r0 = 0, pc = 0;
+  int R = 0, C = 0, K = 0, n = 0;
+};
+
 template <int PB>
 __global__ __launch_bounds__(256, 2) void panel_step_kernel(PanelGroup grp, int64_t ld, int64_t j0, int n, int64_t k,
-                                                            int64_t n_potrf, int64_t r0, int R, int C, int64_t pc,
-                                                            int K, int64_t upc, int64_t copy_j0) {
+                                                            int64_t n_potrf, Update u, int64_t upc,
+                                                            int64_t copy_j0) {
   __shared__ __align__(16) union {
     PotrfLds<float, PB> p;
-    WideLds s;
+    SplitLds s;
   } sm;
   const PanelPtrs& p = grp.p[blockIdx.y];
-  const int64_t n_upd = gridDim.x - n_potrf - (p.copy ? 1 : 0);
   if (p.copy && (int64_t)blockIdx.x == gridDim.x - 1) {
     stage_to_w<float, PB>(p.w, ld, copy_j0, PB, p.copy);
     return;
@@ -1033,8 +963,8 @@ __global__ __launch_bounds__(256, 2) void panel_step_kernel(PanelGroup grp, int6
     return;
   }
   int bi, bj;
-  trapezoid_block(xcd_contiguous(blockIdx.x - n_potrf, n_upd), (C + WB - 1) / WB, bi, bj);
-  syrk_wide_block(sm.s, p.w, ld, r0, R, C, pc, K, bi, bj);
+  trapezoid_block(xcd_contiguous(blockIdx.x - n_potrf, u.n), (u.R + WB - 1) / WB, (u.C + WB - 1) / WB, bi, bj);
+  syrk_wide_block(sm.s, p.w, ld, u.r0, u.R, u.C, u.pc, u.K, bi, bj);
 }
 
 // Launch sequence of the blocked Cholesky of W (k x k) in place over the panels [col_begin, col_end)
@@ -1054,9 +984,8 @@ __global__ __launch_bounds__(256, 2) void panel_step_kernel(PanelGroup grp, int6
 template <typename T>
 struct CholeskyRun {
   static constexpr int PB = LdlBlock<T>::PB;
-  // strip width of the two-level fp32 path: 1024 columns from k = 8192, 512 below (both 8192 factors 10.53 ms
-  // with 256, 10.32 with 512, 10.16-10.25 with 1024; 14336 + 4096: 23.14 with 512, 22.72-22.90 with 1024; 4096:
-  // 3.15 with 256, 3.12 with 512, 3.22 with 1024).  The inverse's split points (multiples of 1024,
+  // strip width of the two-level fp32 path: 1024 columns from k = 8192, 512 below (14336 + 4096: 18.55 ms with
+  // 1024, 18.8 with 512, 19.5 with 256; both 8192 factors 7.91 with 1024 and 512; 4096: 2.38 with 512).  The inverse's split points (multiples of 1024,
   // trtri_split) must be strip boundaries: the strip launch of the panel before one copies that panel's
   // diagonal block into W, which the inverse's first part reads from beside the rest of the chain.
   static constexpr int64_t SW_SMALL = 8 * PB, SW_LARGE = 16 * PB;
@@ -1069,10 +998,9 @@ struct CholeskyRun {
   int64_t col_begin, col_end, j0;
   int64_t sw;  // strip width (two-level path)
   bool two_level, fuse, fold, done = false;
-  int64_t pr0 = 0, pC = 0, ppc = 0;  // pending trapezoid update (columns < pC of W[pr0.., pr0..])
+  Update pend{};                     // two levels: the pending trapezoid update
   int64_t pend_j0 = -1;              // plain path: a panel whose staged block is not in W yet (or -1)
   int pend_n = 0;
-  int pK = 0;
   int ng = 1;  // matrices of the group; entry 0 is (w, info, stage)
   T* wg[GROUP_MAX] = {};
   int* infog[GROUP_MAX] = {};
@@ -1146,14 +1074,14 @@ struct CholeskyRun {
   // last panel, one rank-(strip width) update covers everything to its right -- four times the
   // arithmetic per byte of the trailing triangle that a rank-PB update moves.  Look-ahead: the
   // update of the next panel's columns runs on its own (strip kernel), the rest of the update runs
-  // in the launch that factors the next panel.
+  // in the launch that factors the next panel.  (Dealing the blocks beyond the next strip to that strip's other
+  // launches, which leave the matrix cores idle, was slower: a block takes 48 us beside a panel's 22, so that every
+  // launch with a share of them waits for two rounds; 14336 + 4096 18.6 -> 20.6 ms.)
   int step_two_level() {
     int rc;
     const int n = k - j0 < PB ? (int)(k - j0) : PB;
     const int64_t rest = k - j0 - PB;
     const int64_t blocks = rest > 0 ? (cdiv(rest, 64) < 256 ? cdiv(rest, 64) : 256) : 1;
-    const int64_t pR = pC > 0 ? k - pr0 : 0;
-    const int64_t upd = pC > 0 ? trapezoid_blocks(pR, pC) : 0;
     // the strip of panel j0: [s_lo, s_hi)
     const int64_t s_al = j0 / sw * sw;
     const int64_t s_lo = s_al > col_begin ? s_al : col_begin;
@@ -1166,11 +1094,8 @@ struct CholeskyRun {
     for (int f = 0; f < ng; ++f)
       pp.p[f] = PanelPtrs{(float*)wg[f], infog[f], (float*)slot(j0, f),
                           in_strip ? (const float*)slot(j0 - PB, f) : nullptr};
-    hipLaunchKernelGGL((panel_step_kernel<PB>), dim3((unsigned)(blocks + upd + (in_strip ? 1 : 0)), ny), dim3(256), 0,
-                       stream, pp, k, j0, n, k, blocks, pr0, (int)pR, (int)pC, ppc, pK,
-                       in_strip ? j0 - PB : (int64_t)-1, j0 - PB);
-    if ((rc = (int)hipGetLastError())) return rc;
-    pC = 0;
+    if ((rc = launch_step(pp, n, blocks, in_strip))) return rc;
+    pend.n = 0;
     if (rest <= 0) {  // the last panel: its staged block into W on its own
       for (unsigned f = 0; f < ny; ++f) {
         hipLaunchKernelGGL((stage_to_w_kernel<float, PB>), dim3(1), dim3(256), 0, stream, pp.p[f].w, k, j0, n,
@@ -1190,15 +1115,28 @@ struct CholeskyRun {
       if ((rc = (int)hipGetLastError())) return rc;
     }
     // the rest: the strip's later columns, or everything to the right at a strip's end
-    const int64_t r0 = j0 + 2 * PB, R = rest - PB;
-    const int64_t C = strip_end ? R : (s_hi - r0 < R ? s_hi - r0 : R);
-    if (R > 0 && C > 0) {
-      pr0 = r0;
-      pC = C;
-      ppc = pc;
-      pK = K;
-    }
+    pend = update(j0 + 2 * PB, strip_end ? k : s_hi, pc, K);
     return 0;
+  }
+
+  // The update of rank K by W's columns pc.. of the lower triangle's columns [r0, c_hi).
+  Update update(int64_t r0, int64_t c_hi, int64_t pc, int K) const {
+    Update u{};
+    if (c_hi > k) c_hi = k;
+    if (r0 >= c_hi) return u;
+    u.r0 = r0;
+    u.pc = pc;
+    u.R = (int)(k - r0);
+    u.C = (int)(c_hi - r0);
+    u.K = K;
+    u.n = (int)trapezoid_blocks(u.R, u.C);
+    return u;
+  }
+
+  int launch_step(const PanelGroup& pp, int n, int64_t blocks, bool in_strip) const {
+    hipLaunchKernelGGL((panel_step_kernel<PB>), dim3((unsigned)(blocks + pend.n + (in_strip ? 1 : 0)), (unsigned)ng),
+                       dim3(256), 0, stream, pp, k, j0, n, k, blocks, pend, in_strip ? j0 - PB : (int64_t)-1, j0 - PB);
+    return (int)hipGetLastError();
   }
 
   // fp64 (and fp32 with k % 4 != 0): strips of NS columns, left-looking inside a strip, right-looking
@@ -1300,15 +1238,12 @@ struct CholeskyRun {
   int finish() {
     if (const int rc = flush_staged()) return rc;
     if constexpr (sizeof(T) == 4) {
-      if (pC <= 0) return 0;
-      const int64_t pR = k - pr0;
+      if (!pend.n) return 0;
       PanelGroup pp{};
       for (int f = 0; f < ng; ++f) pp.p[f] = PanelPtrs{(float*)wg[f], infog[f], (float*)stageg[f], nullptr};
-      hipLaunchKernelGGL((panel_step_kernel<PB>), dim3((unsigned)trapezoid_blocks(pR, pC), (unsigned)ng), dim3(256),
-                         0, stream, pp, k, (int64_t)0, 0, k, (int64_t)0, pr0, (int)pR, (int)pC, ppc, pK, (int64_t)-1,
-                         (int64_t)0);
-      pC = 0;
-      return (int)hipGetLastError();
+      const int rc = launch_step(pp, 0, 0, false);
+      pend.n = 0;
+      return rc;
     }
     return 0;
   }

@@ -36,7 +36,7 @@ int gptq2d_gemm(const GemmProblem<T>& p, hipStream_t stream);
 // operand whose other triangle holds zeros: tri = 1: B (B(k, j) = 0 for k < j), tri = 2: A
 // (A(i, k) = 0 for k > i), 0: dense.  A: M x K (row stride lda, batch stride sa), B: K x N, D: M x N.
 // On MFMA, skipping the k-tiles that meet only the zero triangle (trmm_mfma.hip).  Needs K, N, lda,
-// ldb, sa, sb multiples of 4, A and B on 16-byte boundaries and each operand under 2^29 elements;
+// ldb, sa, sb multiples of 4, ldb >= N, A and B on 16-byte boundaries and each operand under 2^29 elements;
 // returns GPTQ2D_EUNSUPPORTED otherwise (nothing launched).
 struct TriGemm {
   int64_t M, N, K, batch;

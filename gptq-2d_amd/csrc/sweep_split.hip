@@ -27,6 +27,7 @@
 #include "diag_sweep.h"
 #include "flush_items.h"
 #include "profile.h"
+#include "split_mma.h"
 #include "tile_sweep.h"
 
 template <typename T>
@@ -35,7 +36,6 @@ double gptq2d_flush_flops(int64_t m, int64_t n, int64_t P, int64_t Q, int64_t s0
 
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int64_t HB = 3 * 64 * 16;  // bytes of a 16-deep half block: three pieces of 64 lanes x 16 bytes
 
@@ -85,36 +85,11 @@ __global__ void batch_offsets_kernel(int64_t* table, int64_t B, BatchMap lmap, B
   table[4 * b + 3] = zmap.offset(b);
 }
 
-// x = h + m + l in bf16 pieces, eight values at once.
-__device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&p)[3]) {
-#pragma unroll
-  for (int s = 0; s < 8; ++s) {
-    const __bf16 h = (__bf16)x[s];
-    const float r = x[s] - (float)h;
-    const __bf16 m = (__bf16)r;
-    p[0][s] = h;
-    p[1][s] = m;
-    p[2][s] = (__bf16)(r - (float)m);
-  }
-}
-
 __device__ __forceinline__ void store_half(char* half, int lane, const float (&x)[8]) {
   bf16x8 p[3];
   split8(x, p);
 #pragma unroll
   for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x8*>(half + 1024 * k + 16 * lane) = p[k];
-}
-
-// The six piece products of a 16-deep half, smallest first.
-constexpr int NPROD = 6;
-__device__ constexpr int prod_a[NPROD] = {2, 0, 1, 1, 0, 0};
-__device__ constexpr int prod_b[NPROD] = {0, 2, 1, 0, 1, 0};
-
-__device__ __forceinline__ bool any_nonfinite(const floatx16& acc) {
-  float s = 0.f;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) s = __builtin_fmaf(acc[r], 0.f, s);
-  return __builtin_amdgcn_ballot_w64(!(s == 0.f)) != 0;
 }
 
 // Row I and column t < I of the k-th block in the packed order of a strict lower triangle (row I at I (I - 1) / 2).

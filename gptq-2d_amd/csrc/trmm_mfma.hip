@@ -1,4 +1,4 @@
-// Row-major fp32 products with one lower triangular operand, on MFMA (v_mfma_f32_32x32x2_f32): the
+// Row-major fp32 products with one lower triangular operand, on split operands (split_mma.h): the
 // levels of the LDL's triangular inverse (ldl.hip), where every product multiplies an inverted
 // diagonal block, lower triangular with its upper triangle cleared to zeros.
 //
@@ -10,46 +10,33 @@
 // halves the arithmetic of a triangular product.  The boundary k-tiles (where the triangle's edge
 // crosses the block) are multiplied in full: the zeros stored there make the result exact.
 //
-// One workgroup per 128 x 128 block of D, four waves of 64 x 64 (2 x 2 MFMA tiles).  The K loop
-// walks k-tiles of 32; both panels are loaded one k-tile ahead straight into LDS (buffer loads with
-// the LDS destination bit), double-buffered, one barrier per k-tile -- the scheme of the sweep's
-// outer flush (flush_mfma.hip), with the same LDS layouts: A (128 rows x 32 k) with its 16-byte
-// k-quads XOR-swizzled by row (quad_swizzle, lds_dma.h), B (32 k-rows x 128 columns) padded by 4 floats per
-// two k-rows.
+// One workgroup per 128 x 128 block of D, four waves of 64 x 64.  A's k runs along a row: a thread's eight values
+// of a k-tile are two 128-bit loads; B's runs down a column: eight loads, coalesced along the columns.
 // Loads past the matrices return zeros (buffer range checks), so ragged edges need no branches.
 #include "common.h"
 #include "lds_dma.h"
 #include "linalg.h"
-
-#include <type_traits>
+#include "split_mma.h"
 
 namespace {
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-
 constexpr int TB = 128;  // block edge
-constexpr int KT = 32;   // k-tile depth
-constexpr int BPAD = 4;  // B panel: floats of padding per 256 (two k-rows of 128 columns)
-constexpr int BSZ = TB * KT + TB * KT / 256 * BPAD;
-
-struct TrmmLds {
-  float a[2][TB * KT];
-  float b[2][BSZ];
-};
+constexpr int KT = 16;   // k-tile depth
+constexpr int BAND = 8;  // block rows whose blocks are numbered column by column: 64 blocks in flight on an XCD share
+                         // 8 panels of either operand
 
 __global__ __launch_bounds__(256, 2) void tri_gemm_kernel(TriGemm g, int64_t nbn) {
-  __shared__ __align__(16) TrmmLds sm;
-  // blocks renumbered so that each XCD (own L2) runs a contiguous share: neighbouring blocks of a
-  // block row share their A panels
-  const int64_t nwg = gridDim.x, w = blockIdx.x;
-  const int64_t base = nwg / 8, extra = nwg % 8, xcd = w % 8;
-  const int64_t lin = xcd * base + (xcd < extra ? xcd : extra) + w / 8;
-  int bi = (int)(lin / nbn);
-  const int bj = (int)(lin % nbn);
+  __shared__ __align__(16) SplitLds sm;
+  const int nbm = (int)((g.M + TB - 1) / TB);
+  const int64_t lin = xcd_contiguous(blockIdx.x, gridDim.x);
+  const int band0 = (int)(lin / (nbn * BAND)) * BAND, rows = nbm - band0 < BAND ? nbm - band0 : BAND;
+  const int64_t at = lin - (int64_t)band0 * nbn;
+  int bi = band0 + (int)(at % rows);
+  const int bj = (int)(at / rows);
   if (g.tri == 2) {
     // a block row's k range grows with its index: rows taken as 0, last, 1, last - 1, ... so that
     // every XCD's contiguous share mixes long and short rows
-    const int nbm = (int)((g.M + TB - 1) / TB), q = bi;
+    const int q = bi;
     bi = (q & 1) ? nbm - 1 - (q >> 1) : (q >> 1);
   }
   const int I0 = bi * TB, J0 = bj * TB;
@@ -62,113 +49,34 @@ __global__ __launch_bounds__(256, 2) void tri_gemm_kernel(TriGemm g, int64_t nbn
   const int nkt = (K + KT - 1) / KT;
   int t_lo = 0, t_hi = nkt;
   if (g.tri == 1) t_lo = J0 / KT;
-  if (g.tri == 2) t_hi = (I0 + TB + KT - 1) / KT < nkt ? (I0 + TB + KT - 1) / KT : nkt;
+  if (g.tri == 2) t_hi = (I0 + TB) / KT < nkt ? (I0 + TB) / KT : nkt;
 
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // buffer resources based at the block's rows of A and, per k-tile, at the k-tile's rows of B, so that every
-  // byte offset stays below 128 rows of lda (A) or 32 rows of ldb (B) floats at any operand size
+  // byte offset stays below 128 rows of lda (A) or 16 rows of ldb (B) floats at any operand size
   const int arows = M - I0 < TB ? M - I0 : TB;
   const __amdgpu_buffer_rsrc_t ra = matrix_rsrc(A + (int64_t)I0 * lda, (int64_t)(arows - 1) * lda + K);
-  auto b_rsrc = [&](int k0) {
-    const int krows = K - k0 < KT ? K - k0 : KT;
-    return matrix_rsrc(B + (int64_t)k0 * ldb + J0, (int64_t)(krows - 1) * ldb + (N - J0));
+  const int row = 32 * wave + li;  // A's row and B's column staged by this thread
+  const bool arow = row < arows, bcol = J0 + row < N;
+  const int aoff = (row * lda + 8 * hh) * 4;
+  int boff[8];  // rows past K lie past the resource's extent (ldb >= N)
+#pragma unroll
+  for (int s = 0; s < 8; ++s) boff[s] = bcol ? ((8 * hh + s) * ldb + row) * 4 : OOB;
+  auto load_a = [&](int t, float (&x)[8]) {
+    const int k = t * KT + 8 * hh;
+    load_row8(ra, arow && k < K ? aoff : OOB, arow && k + 4 < K ? aoff + 16 : OOB, 64 * t, x);
   };
-
-  // per-lane staging of the wave's four 128-bit loads per panel and k-tile: A row `arow`, k-quad
-  // akq (swizzled); B k-row bk, columns bcol .. bcol + 3
-  int aoff[4], akk[4], boff[4], bk[4];
+  auto load_b = [&](int t, float (&x)[8]) {
+    const int k0 = t * KT, krows = K - k0 < KT ? K - k0 : KT;
+    const __amdgpu_buffer_rsrc_t rb = matrix_rsrc(B + (int64_t)k0 * ldb + J0, (int64_t)(krows - 1) * ldb + (N - J0));
 #pragma unroll
-  for (int x = 0; x < 4; ++x) {
-    const int f = (wave + 4 * x) * 256 + 4 * lane;
-    const int row = f >> 5, kq = ((f >> 2) & 7) ^ quad_swizzle(row);
-    akk[x] = 4 * kq;
-    aoff[x] = row < arows ? (row * lda + akk[x]) * 4 : OOB;
-    bk[x] = f >> 7;
-    const int col = f & (TB - 1);
-    boff[x] = J0 + col < N ? (bk[x] * ldb + col) * 4 : OOB;
-  }
-  // a block whose rows and columns all lie inside D takes its interior k-tiles (every lane in range) with
-  // the k offset in the loads' scalar field: no vector instruction beside the MFMA bursts
-  const bool full = I0 + TB <= M && J0 + TB <= N;
-  auto issue = [&](int t, int buf) {
-    const int k0 = t * KT;
-    const __amdgpu_buffer_rsrc_t rb = b_rsrc(k0);
-    if (full && k0 + KT <= K) {
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        const int f0 = (wave + 4 * x) * 256;
-        dma_load_so<4>(ra, &sm.a[buf][f0], aoff[x], k0 * 4);
-        dma_load_so<4>(rb, &sm.b[buf][f0 + f0 / 256 * BPAD], boff[x], 0);
-      }
-      return;
-    }
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const int f0 = (wave + 4 * x) * 256;
-      const bool aok = aoff[x] != OOB && k0 + akk[x] < K;
-      dma_load<4>(ra, &sm.a[buf][f0], aok ? aoff[x] + k0 * 4 : OOB);
-      const bool bok = boff[x] != OOB && k0 + bk[x] < K;
-      dma_load<4>(rb, &sm.b[buf][f0 + f0 / 256 * BPAD], bok ? boff[x] : OOB);
-    }
+    for (int s = 0; s < 8; ++s)
+      x[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, boff[s], 0, 0));
   };
-
-  floatx16 acc[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int d = 0; d < 2; ++d)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[a][d][r] = 0.f;
-
-  // fragments: A tile a, k-quad 4 hh + v of row 64 wy + 32 a + li; B tile d, k = 16 hh + s, column
-  // 64 wx + 32 d + li -- the k of MFMA s is 16 hh + s for both operands
   const int wy = wave >> 1, wx = wave & 1;
-  const int a_base = (64 * wy + li) * KT, sw = quad_swizzle(li);
-  const int b_base = 16 * hh * TB + 64 * wx + li + 16 * hh * TB / 256 * BPAD;
-  auto step = [&](int t, auto cur_c) {
-    constexpr int cur = decltype(cur_c)::value;
-    __syncthreads();  // buffer cur is complete; buffer 1 - cur is no longer read
-    if (t + 1 < t_hi) issue(t + 1, 1 - cur);
-    const float* as = &sm.a[cur][a_base];
-    const float* bs = &sm.b[cur][b_base];
-    float4 fa[2][2];
-    float fb[2][2][4];
-    auto frag = [&](int v, int slot) {
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-        fa[slot][a] = *reinterpret_cast<const float4*>(as + a * 32 * KT + 4 * ((4 * hh + v) ^ sw));
-#pragma unroll
-      for (int d = 0; d < 2; ++d)
-#pragma unroll
-        for (int s2 = 0; s2 < 4; ++s2) {
-          const int s = 4 * v + s2;
-          fb[slot][d][s2] = bs[32 * d + s * TB + s * TB / 256 * BPAD];
-        }
-    };
-    frag(0, 0);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      if (v < 3) frag(v + 1, (v + 1) & 1);
-#pragma unroll
-      for (int s2 = 0; s2 < 4; ++s2)
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-          for (int d = 0; d < 2; ++d)
-            acc[a][d] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[v & 1][a][s2], fb[v & 1][d][s2], acc[a][d], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    wait_dma();  // this wave's loads of k-tile t + 1 have landed before the next barrier
-  };
-  if (t_lo < t_hi) {
-    issue(t_lo, 0);
-    wait_dma();
-    for (int t = t_lo; t < t_hi; t += 2) {
-      step(t, std::integral_constant<int, 0>{});
-      if (t + 1 < t_hi) step(t + 1, std::integral_constant<int, 1>{});
-    }
-  }
+  floatx16 acc[2][2];
+  split_block_product(sm, t_lo, t_hi, acc, load_a, load_b);
   const float alpha = g.alpha;
 #pragma unroll
   for (int a = 0; a < 2; ++a)
@@ -199,7 +107,7 @@ int gptq2d_tri_gemm_f32(const TriGemm& g, hipStream_t stream) {
     return GPTQ2D_EUNSUPPORTED;
   // 32-bit byte offsets inside a block's 128 rows of A (plus K) and a k-tile's 32 rows of B (plus N)
   const int64_t lim = (int64_t)1 << 29;
-  if (TB * g.lda + g.K >= lim || KT * g.ldb + g.N >= lim || g.M >= lim || g.N >= lim || g.K >= lim || g.K == 0)
+  if (TB * g.lda + g.K >= lim || 32 * g.ldb + g.N >= lim || g.M >= lim || g.N >= lim || g.K >= lim || g.K == 0 || g.ldb < g.N)
     return GPTQ2D_EUNSUPPORTED;
   const int64_t nbm = (g.M + TB - 1) / TB, nbn = (g.N + TB - 1) / TB;
   if (nbm * nbn > 0x7fffffff) return GPTQ2D_EUNSUPPORTED;
