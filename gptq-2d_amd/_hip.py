@@ -116,15 +116,24 @@ def call_untyped(name: str, *args) -> None:
         raise GPTQ2DError(f"gptq2d_{name} failed with code {rc}")
 
 
-def call(name: str, dtype: torch.dtype, *args) -> None:
-    """Call ``gptq2d_<name>_<f32|f64>`` and raise on a non-zero return code."""
+def function(name: str, dtype: torch.dtype):
+    """``gptq2d_<name>_<f32|f64>`` as a callable that raises on a non-zero return code."""
     suffix = {torch.float32: "f32", torch.float64: "f64"}.get(dtype)
     if suffix is None:
         raise GPTQ2DError(f"unsupported dtype {dtype}")
     fn = getattr(lib(), f"gptq2d_{name}_{suffix}")
-    rc = fn(*args)
-    if rc != 0:
-        raise GPTQ2DError(f"gptq2d_{name}_{suffix} failed with code {rc}")
+
+    def checked(*args) -> None:
+        rc = fn(*args)
+        if rc != 0:
+            raise GPTQ2DError(f"gptq2d_{name}_{suffix} failed with code {rc}")
+
+    return checked
+
+
+def call(name: str, dtype: torch.dtype, *args) -> None:
+    """Call ``gptq2d_<name>_<f32|f64>`` and raise on a non-zero return code."""
+    function(name, dtype)(*args)
 
 
 # Kernel classes of the launch profiler (csrc/profile.h).
