@@ -68,15 +68,34 @@ __device__ __forceinline__ T quantize_absmax_entry(T yv, T sv, T qmin, T qmax) {
 // Thread (g, c) = (tid / 32, tid % 32) owns column c of rows 4g .. 4g + 3; a row is the 32 lanes of one
 // half-wave, so the abs-max of a super-entry row is a half-wave reduction.
 
-// Maximum over the 32 lanes of each half-wave (all of them receive it).
+// Maximum over the 32 lanes of each half-wave (all of them receive it).  fp32: by exchanges of lanes in the vector
+// registers (quad permutes, mirrors of 8 and 16 lanes, the swap of 16-lane rows), 10 instructions; five shuffles
+// through LDS are 65 clocks each on the chain of every row.
 template <typename T>
 __device__ __forceinline__ T halfwave_max(T v) {
+  if constexpr (sizeof(T) == 4) {
+    auto with = [&](auto ctrl_c) {
+      const T o = __builtin_bit_cast(
+          T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), decltype(ctrl_c)::value, 0xf, 0xf, true));
+      v = o > v ? o : v;
+    };
+    with(std::integral_constant<int, 0xB1>{});   // lane ^ 1
+    with(std::integral_constant<int, 0x4E>{});   // lane ^ 2
+    with(std::integral_constant<int, 0x141>{});  // the other quad of 8 lanes
+    with(std::integral_constant<int, 0x140>{});  // the other half of 16
+    const unsigned u = __builtin_bit_cast(unsigned, v);
+    const auto rows = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const unsigned r0 = rows[0], r1 = rows[1];
+    const T a = __builtin_bit_cast(T, r0), b = __builtin_bit_cast(T, r1);
+    return b > a ? b : a;
+  } else {
 #pragma unroll
-  for (int k = 16; k >= 1; k >>= 1) {
-    const T o = __shfl_xor(v, k, 32);
-    v = o > v ? o : v;
+    for (int k = 16; k >= 1; k >>= 1) {
+      const T o = __shfl_xor(v, k, 32);
+      v = o > v ? o : v;
+    }
+    return v;
   }
-  return v;
 }
 
 // The rows' quantizer inputs (affine: scale and zero point; forced: the values), read from global memory
@@ -115,7 +134,7 @@ __device__ __forceinline__ void sweep_rows(T* ys, int ysp, T* cs, int csp, const
                                            int esp, const RowInputs<T, KIND>& in, T* __restrict__ y,
                                            T* __restrict__ c, T* __restrict__ e, const QSpec<T>& qs, int64_t m,
                                            int64_t n, int64_t i0, int64_t j0, int64_t mat) {
-  const int cc = threadIdx.x & 31, g = threadIdx.x >> 5;
+  const int cc = threadIdx.x & 31, g = threadIdx.x >> 5, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rows_in = m - i0 < TR ? (int)(m - i0) : TR;  // the super-entries span the tile's columns
   T Y[4], C[4], D[4], E[4];
 #pragma unroll
@@ -127,35 +146,37 @@ __device__ __forceinline__ void sweep_rows(T* ys, int ysp, T* cs, int csp, const
   const T qmin = qs.qmin, qmax = qs.qmax, half = (qs.qmax - qs.qmin) / T(2);
   auto step = [&](auto r_c) __attribute__((always_inline)) {
     constexpr int r = decltype(r_c)::value, slot = r & 3;
-    const bool own = g == (r >> 2) && r < rows_in;
-    const T yv = Y[slot] + D[slot];
-    T z, sc = T(1);
-    if constexpr (KIND == Q_ABSMAX) {
-      // scale from the row's current abs max (a NaN entry counts as 0, as in the plug-in's comparison
-      // loop), rounded to the 16-bit type through fp32, 0 -> 1; the reduction runs on every lane
-      const T a = own ? __builtin_fmax(__builtin_fabs(yv), T(0)) : T(0);
-      const T amax = halfwave_max(a);
-      sc = round_scale16(amax / half, qs.dtype16);
-      sc = sc == T(0) ? T(1) : sc;
-      z = quantize_absmax_entry(yv, sc, qmin, qmax);
-    } else if constexpr (KIND == Q_AFFINE) {
-      // the dequantized value rounded on its own, before the error z - y (no contraction into it)
-      z = quantize_entry_div(yv, in.s[slot], in.z[slot], qmin, qmax);
-    } else if constexpr (KIND == Q_FORCED) {
-      z = in.s[slot];
-    } else {
-      z = round_even(yv);
-    }
-    const T ev = z - yv;
-    const T cf = (C[slot] + D[slot]) + ev;
-    if (own) {
-      Y[slot] = z;
-      E[slot] = ev;
-      C[slot] = cf;
-      es[r * esp + cc] = ev;
-      if constexpr (YPRE) qs.ypre[mat + (i0 + r) * n + j0 + cc] = yv;
+    if (wave == (r >> 3)) {  // the wave that holds the row; the others wait for its errors
+      const bool own = g == (r >> 2) && r < rows_in;
+      const T yv = Y[slot] + D[slot];
+      T z, sc = T(1);
       if constexpr (KIND == Q_ABSMAX) {
-        if (qs.sout) qs.sout[mat + (i0 + r) * n + j0 + cc] = sc;
+        // scale from the row's current abs max (a NaN entry counts as 0, as in the plug-in's comparison
+        // loop), rounded to the 16-bit type through fp32, 0 -> 1; the reduction runs on every lane
+        const T a = own ? __builtin_fmax(__builtin_fabs(yv), T(0)) : T(0);
+        const T amax = halfwave_max(a);
+        sc = round_scale16(amax / half, qs.dtype16);
+        sc = sc == T(0) ? T(1) : sc;
+        z = quantize_absmax_entry(yv, sc, qmin, qmax);
+      } else if constexpr (KIND == Q_AFFINE) {
+        // the dequantized value rounded on its own, before the error z - y (no contraction into it)
+        z = quantize_entry_div(yv, in.s[slot], in.z[slot], qmin, qmax);
+      } else if constexpr (KIND == Q_FORCED) {
+        z = in.s[slot];
+      } else {
+        z = round_even(yv);
+      }
+      const T ev = z - yv;
+      const T cf = (C[slot] + D[slot]) + ev;
+      if (own) {
+        Y[slot] = z;
+        E[slot] = ev;
+        C[slot] = cf;
+        es[r * esp + cc] = ev;
+        if constexpr (YPRE) qs.ypre[mat + (i0 + r) * n + j0 + cc] = yv;
+        if constexpr (KIND == Q_ABSMAX) {
+          if (qs.sout) qs.sout[mat + (i0 + r) * n + j0 + cc] = sc;
+        }
       }
     }
     if constexpr (r + 1 < TR) {
