@@ -28,7 +28,6 @@ struct BatchMap {
 
   // Element offset of logical batch b (row-major over shape, last dim fastest).
   __host__ __device__ __forceinline__ int64_t offset(int64_t b) const {
-    if (nd <= 1) return nd == 1 ? b * stride[0] : 0;  // no 64-bit division (hundreds of instructions each)
     int64_t off = 0;
     for (int d = nd - 1; d >= 0; --d) {
       const int64_t sz = shape[d];

@@ -15,13 +15,13 @@
 //      the trailing lower triangle takes the rank-PB update.  fp32 (k % 4 == 0) blocks it on two
 //      levels: strips of 8 panels (16 from k = 8192), where each panel updates only its strip's later
 //      columns and a strip's end brings one update of the whole trailing triangle of the strip's rank
-//      (512 or 1024; MFMA-bound, where
+//      (512 or 1024; bound by the matrix cores, on split bf16 operands (split_mma.h), where
 //      rank-64 updates are bound by moving the triangle through HBM), with a look-ahead of one
 //      panel on the one stream: after a panel, a strip launch updates only the next panel's
 //      columns, and the next panel's factorisation shares one launch (panel_step_kernel) with the
 //      rest of the update, on disjoint columns -- the latency-bound panel runs beside the MFMA
-//      update instead of after it.  fp64 (and fp32 with k % 4 != 0) keep the plain sequence, the
-//      update on gemm.hip.
+//      update instead of after it.  fp64 (and fp32 with k % 4 != 0: a caller can embed
+//      such a matrix in an aligned one, gptq2d_embed_*) keep the plain sequence, the update on gemm.hip.
 //   3. ldl_of_inverse only: C^{-1} in place by recursive doubling.  Diagonal NB blocks are inverted
 //      by one wave each; then for s = NB, 2 NB, ... every pair of inverted s-blocks A^{-1}, D^{-1}
 //      with off-diagonal block B becomes one inverted 2s-block through -D^{-1} (B A^{-1}) -- two
