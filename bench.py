@@ -57,17 +57,18 @@ OUTER_BLOCK_WIDE = 1024
 # HBM bytes per outer-flush launch at OUTER_BLOCK on the headline layer, mean over a step's 21
 # launches: rocprofv3 FETCH_SIZE and WRITE_SIZE passes (one counter per run) over this benchmark,
 # each scaled by what the same counter reads for a plain 256 MiB copy kernel in the same run
-# (x1.9997 and x1.0000).  Counters cannot be read inside the timed run, so the figure is the
-# measured one, with the command and per-kernel values in profiles/flush_traffic_H_int4.md; the
-# algorithmic minimum (every operand once) is FLUSH_ALGORITHMIC_BYTES.
-FLUSH_TRAFFIC_BYTES = 1.718e9
+# (x1.9998 and x1.0000).  Counters cannot be read inside the timed run, so the figure is the
+# measured one, with the command and per-kernel values in profiles/split_engine_kernels.md; the
+# algorithmic minimum (every operand once, in fp32: split operands are 1.5 times as long) is
+# FLUSH_ALGORITHMIC_BYTES.
+FLUSH_TRAFFIC_BYTES = 1.530e9
 FLUSH_ALGORITHMIC_BYTES = 0.489e9
 # The same two counter passes give the other kernels' HBM bytes, from which the line reports their achieved
 # HBM rates against the live timings: a tile-stage launch at OUTER_BLOCK on the headline layer (FETCH_SIZE
-# 13703.9 KiB x 1.9997 + WRITE_SIZE 2479.6 KiB, mean over a step's 511 launches) and one Viterbi call of the
-# benchmark's search (FETCH_SIZE 132672.3 KiB x 2.0 + WRITE_SIZE 2081294.9 KiB: its step-minimum history);
-# profiles/flush_traffic_H_int4.md, profiles/counters_H_int4.md and profiles/viterbi_hyb_counters.md.
-TILE_STAGE_TRAFFIC_BYTES = 30.60e6
+# 19196.2 KiB x 1.9998 + WRITE_SIZE 4018.6 KiB, mean over a step's 511 launches; profiles/split_engine_kernels.md)
+# and one Viterbi call of the benchmark's search (FETCH_SIZE 132672.3 KiB x 2.0 + WRITE_SIZE 2081294.9 KiB: its
+# step-minimum history; profiles/viterbi_hyb_counters.md).
+TILE_STAGE_TRAFFIC_BYTES = 43.42e6
 VITERBI_TRAFFIC_BYTES = 2.403e9
 # fp32 VALU operations per trellis state evaluation of the plain search: 2 sub, 2 mul, 1 add (the squared
 # distance), 1 add (the predecessor group's minimum), 1 min.
@@ -224,7 +225,7 @@ def _tile_stage_line(sweep_ms, flush_ms, m, n):
         "traffic_unit": "B per launch (rocprofv3, copy-calibrated)",
         "achieved_gbs": round(TILE_STAGE_TRAFFIC_BYTES / (us * 1e-6) / 1e9, 1) if known else None,
         "peak_gbs": HBM_PEAK_GBS,
-        "bound": "latency (63 dependent in-tile steps per launch, one barrier each)",
+        "bound": "latency (63 dependent in-tile steps per launch)",
     }
 
 
