@@ -46,13 +46,13 @@ VALU_FP32_OPS_PEAK = 39.3e12
 # Outer block of the fused sweep, in antidiagonals (24 tile stages).  A longer outer block moves
 # more of the cross-tile feedback into the few large outer flushes, which run closest to the MFMA
 # peak, at the price of more in-block prep work per tile stage (whose MFMA pulls slow the in-tile
-# sweeps beside them); sweep of the 8192^2 layer on one MI355X, best of four: 512 -> 19.7 ms,
-# 640 -> 19.1, 704 -> 19.0, 768 -> 19.1, 832 -> 19.1, 1024 -> 19.6, 1536 -> 21.4, 2048 -> 23.9 ms.
+# sweeps beside them); sweep of the 8192^2 layer on one MI355X: 512 -> 13.9 ms, 640 -> 13.7,
+# 768 -> 13.7, 896 -> 13.9, 1024 -> 14.0, 1536 -> 15.6 ms.
 # It changes the order of the fp32 additions only, not the algorithm.
 OUTER_BLOCK = 768
 # The 8192 x 28672 layers of C5a (1 x 32 super-entry rows, and the three-sided D-sided form) sweep fastest with
-# longer blocks: C5a 768 -> 94.4 ms, 1024 -> 94.0, 1280 -> 95.2-95.9, 1536 -> 97.6, 2048 -> 104.3 (2 x 2-tile
-# outer flushes; with 4 x 4 ones 1280 had been best at 97.6).
+# longer blocks for C5a (on the fp32 MFMA: 768 -> 94.4 ms, 1024 -> 94.0, 1280 -> 95.2-95.9, 1536 -> 97.6,
+# 2048 -> 104.3).
 OUTER_BLOCK_WIDE = 1024
 # HBM bytes per outer-flush launch at OUTER_BLOCK on the headline layer, mean over a step's 21
 # launches: rocprofv3 FETCH_SIZE and WRITE_SIZE passes (one counter per run) over this benchmark,
