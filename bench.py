@@ -51,7 +51,7 @@ VALU_FP32_OPS_PEAK = 39.3e12
 # It changes the order of the fp32 additions only, not the algorithm.
 OUTER_BLOCK = 768
 # The 8192 x 28672 layers of C5a (1 x 32 super-entry rows, and the three-sided D-sided form) sweep fastest with
-# longer blocks for C5a (on the fp32 MFMA: 768 -> 94.4 ms, 1024 -> 94.0, 1280 -> 95.2-95.9, 1536 -> 97.6,
+# longer blocks (on the fp32 MFMA: 768 -> 94.4 ms, 1024 -> 94.0, 1280 -> 95.2-95.9, 1536 -> 97.6,
 # 2048 -> 104.3).
 OUTER_BLOCK_WIDE = 1024
 # HBM bytes per outer-flush launch at OUTER_BLOCK on the headline layer, mean over a step's 21
