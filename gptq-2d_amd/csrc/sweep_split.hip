@@ -320,6 +320,7 @@ __global__ __launch_bounds__(DTHREADS, 2) void tile_stage_split_kernel(StageArgs
       bv[p] = *reinterpret_cast<const bf16x8*>(pb + ch * HB + 1024 * p + 16 * lane);
     }
   }
+  static_assert(DTHREADS / TR == 16, "entry k of a thread lies in the tile's rows 16 k .. 16 k + 15");
   float yo[NQ], co[NQ], so[NQ], zo[NQ], lo[NQ], uo[NQ], pu[NQ];
   {
     auto rsrc = [](const float* p) {
@@ -331,8 +332,7 @@ __global__ __launch_bounds__(DTHREADS, 2) void tile_stage_split_kernel(StageArgs
     const int64_t corner = (int64_t)i0 * n + j0;
     const __amdgpu_buffer_rsrc_t ry = rsrc(g.y + at), rc = rsrc(g.c + at);
     const __amdgpu_buffer_rsrc_t rl = rsrc(g.l + off.l + (int64_t)i0 * m + i0);
-    const __amdgpu_buffer_rsrc_t ru = rsrc(KR ? g.kr.q : g.u + off.u + (int64_t)j0 * n + j0);
-    const __amdgpu_buffer_rsrc_t rp = rsrc(KR ? g.kr.p : nullptr);
+    const __amdgpu_buffer_rsrc_t rt = rsrc(KR ? nullptr : g.u + off.u + (int64_t)j0 * n + j0);
     const __amdgpu_buffer_rsrc_t rs = rsrc(KIND == Q_ROUND ? nullptr : g.scale + off.s + corner);
     const __amdgpu_buffer_rsrc_t rz = rsrc(KIND == Q_AFFINE ? g.zp + off.z + corner : nullptr);
 #pragma unroll
@@ -344,16 +344,21 @@ __global__ __launch_bounds__(DTHREADS, 2) void tile_stage_split_kernel(StageArgs
       yo[k] = load(ry, o);
       co[k] = load(rc, o);
       lo[k] = load(rl, ol);
-      if constexpr (KR) {  // the P entry times the Q entry
-        int ib = 0, iq = 0, jb = 0, jq = 0;
+      if constexpr (KR) {
+        // the P entry times the Q entry.  U's rows j0 + 16 k .. + 15 are 16 rows of Q in one block of P: the resources
+        // are based there, so that no offset exceeds 16 rows of Q (an offset from Q's first entry would not fit 32
+        // bits from nq = 23171 on)
+        int ib, i16, jb = 0, jq = 0;
+        kron_split(g.kr, (unsigned)(j0 / 16 + k), ib, i16);
         if (ou != OOB) {
-          kron_index(g.kr, j0 + r, ib, iq);
           kron_index(g.kr, j0 + cc, jb, jq);
+          ou = (r0 * g.kr.nq + jq) * 4;
         }
-        pu[k] = load(rp, ou != OOB ? (ib * g.kr.np + jb) * 4 : OOB);
-        ou = ou != OOB ? (iq * g.kr.nq + jq) * 4 : OOB;
+        pu[k] = load(rsrc(g.kr.p + (int64_t)ib * g.kr.np), ou != OOB ? jb * 4 : OOB);
+        uo[k] = load(rsrc(g.kr.q + (int64_t)i16 * 16 * g.kr.nq), ou);
+      } else {
+        uo[k] = load(rt, ou);
       }
-      uo[k] = load(ru, ou);
       so[k] = KIND == Q_ROUND ? 0.f : load(rs, o);
       zo[k] = KIND == Q_AFFINE ? load(rz, o) : 0.f;
     }

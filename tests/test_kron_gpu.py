@@ -130,6 +130,26 @@ def test_kron_teacher_forced_values(m, np_, nq, outer):
     assert torch.equal(pre_k, pre_d)
 
 
+@pytest.mark.parametrize("np_,nq", [(1, 23184), (2, 23184), (1, 32784), (2, 32784)])
+def test_kron_large_inner_factor(np_, nq):
+    """Inner factors whose entries lie 2 GiB and 4 GiB behind the first one: every value before rounding equals the
+    explicit product's bit for bit (the in-tile feedback reads Q's diagonal blocks to the last)."""
+    m, n = 36, np_ * nq
+    print(f"kron large {m}x({np_}x{nq})", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(nq + np_)
+    x = 4. * torch.randn(m, n, generator=g, device=DEV)
+    lo, p = _unit_lower(m, 1), _unit_upper(np_, 2)
+    q = torch.randn(nq, nq, generator=g, device=DEV).mul_(.3 / nq ** .5).triu_(1)
+    q.diagonal().fill_(1.)
+    z = torch.round(x)
+    pre_k, pre_d = torch.full_like(x, float("nan")), torch.full_like(x, float("nan"))
+    G.gptq_2d(x, lo, G.KroneckerU(p, q), quantizer=QI.teacher_forced_quantizer, quantizer_inputs=(z, pre_k), fused=True)
+    up = torch.kron(p, q)
+    G.gptq_2d(x, lo, up, quantizer=QI.teacher_forced_quantizer, quantizer_inputs=(z, pre_d), fused=True)
+    del up
+    assert not pre_k.isnan().any() and torch.equal(pre_k, pre_d)
+
+
 def test_kron_resumed_call():
     """Two calls of the C entry point over consecutive outer blocks (stage_begin / stage_end on a block boundary,
     C and E kept between them) equal one call over the whole sweep."""
