@@ -25,6 +25,7 @@ Reference: IST-DASLab/GPTQ-2D gptq_2d.py (entry points :1378-1564, PyTorch sweep
 
 from __future__ import annotations
 
+import ctypes
 import functools
 import math
 from typing import Callable
@@ -48,8 +49,9 @@ class KroneckerU:
     gptq_2d_reference.py:270-294, whose factors the reference never multiplies out).  Entries are read as
     torch.kron(outer, inner) forms them -- every entry of both factors, the product's zeros and diagonal
     included -- so results equal those with ``dense()`` bit for bit.  The fused fp32 engine reads the factors
-    directly (one matrix, no batch; inner size a multiple of 16, sizes multiples of 4); every other path forms
-    ``dense()`` first."""
+    directly (one matrix, no batch; inner size a multiple of 16, sizes multiples of 4) and never forms the product;
+    on split operands it holds the pieces of U's upper triangle in its workspace, 3 n^2 bytes, and where those do
+    not fit it reads the factors throughout.  Every other path forms ``dense()`` (4 n^2 bytes) first."""
 
     def __init__(self, outer: torch.Tensor, inner: torch.Tensor):
         assert outer.dim() == 2 and inner.dim() == 2, "the Kronecker factors must be matrices"
@@ -216,7 +218,8 @@ SPLIT_WORKSPACE_MAX = 32 << 30
 
 
 def _run_split(y, l, u, m, n, batch_shape, spec, outer_block_size, p, q):
-    """The fused fp32 sweep on split operands (gptq2d_sweep_split_f32); False where it does not apply."""
+    """The fused fp32 sweep on split operands (gptq2d_sweep_split_f32); False where it does not apply or its
+    workspace (gptq2d_sweep_split_workspace: 12 bytes an entry of X and 3 k^2 of a factor) cannot be had."""
     if y.dtype != torch.float32 or m >= 1 << 20 or n >= 1 << 20 or batch_shape.numel() > 65535:
         return False
     kron = isinstance(u, KroneckerU)
@@ -226,17 +229,23 @@ def _run_split(y, l, u, m, n, batch_shape, spec, outer_block_size, p, q):
     need = _hip.lib().gptq2d_sweep_split_workspace(m, n, nd, bshape, lstr, ustr)
     if not 0 <= need <= SPLIT_WORKSPACE_MAX:
         return False
-    c, e = torch.empty_like(y), torch.empty_like(y)
-    work = torch.empty(max(need, 16), dtype=torch.uint8, device=y.device)
+    # C, E and the workspace in one allocation; where the device has no room for it, the engine on fp32 operands, which
+    # needs only C and E, takes the call
+    size = -(-4 * y.numel() // 256) * 256
+    try:
+        buf = torch.empty(2 * size + need, dtype=torch.uint8, device=y.device)
+    except torch.OutOfMemoryError:
+        return False
+    c, e, work = (ctypes.c_void_p(buf.data_ptr() + at) for at in (0, size, 2 * size))
     qa, qb = spec["qa"], spec["qb"]
     up, uq = (u.outer, u.inner) if kron else (None, None)
     _hip.call_untyped(
-        "sweep_split_f32", _hip.ptr(y), _hip.ptr(c), _hip.ptr(e), _hip.ptr(l), None if kron else _hip.ptr(u),
+        "sweep_split_f32", _hip.ptr(y), c, e, _hip.ptr(l), None if kron else _hip.ptr(u),
         _hip.ptr(up), _hip.ptr(uq), up.size(0) if kron else 0, uq.size(0) if kron else 0, m, n, p, q, nd, bshape, lstr,
         ustr, spec["kind"], _hip.ptr(qa), _hip.batch_strides(qa, batch_shape) if qa is not None else None, _hip.ptr(qb),
         _hip.batch_strides(qb, batch_shape) if qb is not None else None, spec["qmin"], spec["qmax"],
         spec.get("dtype16", 0), _hip.ptr(spec["ypre"]), _hip.ptr(spec.get("sout")), _outer_tiles(outer_block_size), 0,
-        -1, _hip.ptr(work), work.numel(), _hip.stream(y.device))
+        -1, work, need, _hip.stream(y.device))
     return True
 
 
@@ -419,7 +428,8 @@ def capture_gptq_2d(x, l, u, *, quantizer: Callable | None = None, super_entry_s
 
     Replay inputs must match the examples' shapes, dtypes and devices; they are copied into private
     static buffers.  Out of place a replay returns a clone; in place it copies into x and returns it.
-    One replay callable owns its static buffers and must be used sequentially.
+    One replay callable owns its static buffers and must be used sequentially; it also keeps, until it is deleted,
+    what the captured sweep allocated (C and E, and in fp32 the workspace of the split operands).
     """
     _validate_inputs(x, l, u, inplace, require_cuda=True, super_entry_shape=super_entry_shape or (1, 1))
     assert all(t.is_cuda and t.device == x.device for t in quantizer_inputs), (
