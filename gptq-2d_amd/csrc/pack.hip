@@ -47,17 +47,10 @@ struct IntLayout {
   int64_t zb, zm, zn;
 };
 
-__device__ __forceinline__ int wave_sum(int v) {
-#pragma unroll
-  for (int k = 32; k >= 1; k >>= 1) v += __shfl_xor(v, k, 64);
-  return v;
-}
-
-// Both INT kernels are bound by HBM (the values read or written once, 4 or 8 bytes an entry): a thread takes whole
-// words' codes, or eight, and moves the values 16 bytes at a time (global memory needs only the element's own
-// alignment for that); the scale is read once per row where it does not vary along it, and no thread divides a 64-bit
-// index.  8192^2 fp32 at 4 bits, per-row scale: pack 177 -> 77 us, unpack 192 -> 82 us, together 4.0 TB/s (a code a lane,
-// OR-reduced across lanes, and a 64-bit division per value before).
+// The INT kernels are bound by HBM (the values read or written once, 4 or 8 bytes an entry, and as many bytes again of
+// every scale and zero point that varies along the row), so neighbouring threads read neighbouring 16 bytes of all of
+// them (global memory needs only the element's own alignment for that); a scale or zero point that does not vary along
+// the row is read once per row, and no thread divides a 64-bit index per value.
 //
 // Values j .. j + N - 1 of a row of n; past the row's end 0.
 template <typename T, int N>
@@ -77,73 +70,164 @@ __device__ __forceinline__ void load_values(T (&v)[N], const T* __restrict__ row
   }
 }
 
-// TPR threads per row (64: four rows per workgroup).  BITS 4 or 8: a thread packs the 32 / BITS codes of a word; BITS 0
-// (any width `bits`): the 32 codes of `bits` words.
-template <typename T, int BITS, int TPR>
+// N consecutive values of a field (scale or zero point) of a row from column j on: `fixed` where the row has one.
+template <typename T, int N>
+__device__ __forceinline__ void load_field(T (&v)[N], const T* __restrict__ row, int64_t stride, T fixed, int64_t j,
+                                           int64_t n) {
+  if (stride == 1) {
+    load_values<T, N>(v, row, j, n);
+  } else {
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = stride && j + k < n ? row[(j + k) * stride] : fixed;
+  }
+}
+
+// A row's values, its words, and its scale and zero point (the fields' own values where they vary along it).
+template <typename T>
+struct IntRow {
+  const T *s, *p;
+  T s0, p0;
+  int64_t sn, zn;
+
+  __device__ __forceinline__ IntRow(const IntLayout<T>& lay, int64_t row, int64_t rows, int64_t m,
+                                    int64_t n) {
+    const int64_t b = rows == m ? 0 : row / m, i = rows == m ? row : row % m;
+    s = lay.s + b * lay.sb + i * lay.sm;
+    p = lay.zp ? lay.zp + b * lay.zb + i * lay.zm : nullptr;
+    sn = lay.sn, zn = p ? lay.zn : 0;
+    s0 = sn || n == 0 ? T(0) : *s;
+    p0 = !p || zn || n == 0 ? T(0) : *p;
+  }
+  template <int N>
+  __device__ __forceinline__ void load(T (&sv)[N], T (&pv)[N], int64_t j, int64_t n) const {
+    load_field(sv, s, sn, s0, j, n);
+    load_field(pv, p, zn, p0, j, n);
+  }
+};
+
+// Sum over the TPR threads of a row (in its thread 0).
+template <int TPR>
+__device__ __forceinline__ int row_sum(int v, int (&sums)[4]) {
+#pragma unroll
+  for (int k = (TPR < 64 ? TPR : 64) / 2; k >= 1; k >>= 1) v += __shfl_xor(v, k, 64);
+  if constexpr (TPR == 256) {
+    if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = sums[0] + sums[1] + sums[2] + sums[3];
+  }
+  return v;
+}
+
+// Codes of any width, TPR threads per row.  A thread packs four consecutive values of a chunk of 4 TPR (a whole number
+// of words at any width) into one piece of 4 `bits` bits in LDS, and takes its words of the chunk from the pieces there;
+// the next chunk's values are on their way meanwhile.  4096^2 fp32, 5 bits: one scale per row 23 us, a scale per entry 26,
+// scale and zero point per entry 35 (41, 50 and 77 with a word a lane that gathers its codes, 27, 185 and 576 with 32
+// consecutive values a thread, whose loads touch a cache line each); 16 bits 27, 29, 38; 100000 x 24 at 3 bits 7.7 (94, 133).
+template <typename T, int TPR>
 __global__ __launch_bounds__(256) void int_pack_kernel(const T* __restrict__ z, int64_t rows, int64_t m, int64_t n,
                                                        IntLayout<T> lay, T qmin, T qmax, int bits,
                                                        uint32_t* __restrict__ words, int64_t row_words,
                                                        int32_t* __restrict__ bad) {
+  constexpr int N = 4, CH = N * TPR;
+  __shared__ uint64_t pieces[2][256 / TPR][TPR];
   __shared__ int sums[4];
-  constexpr int N = BITS ? 32 / (BITS ? BITS : 1) : 32;  // codes of a thread's unit
+  const int t = threadIdx.x % TPR;
+  const int64_t at = (int64_t)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
+  const bool live = at < rows;
+  const int64_t row = live ? at : rows - 1;  // the others take part in the barriers only
+  auto sync = [&]() {
+    if constexpr (TPR > 64) {
+      __syncthreads();
+    } else {  // a row's threads are lanes of one wave
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+  };
+  const IntRow<T> f(lay, row, rows, m, n);
+  const T* zr = z + row * n;
+  uint32_t* wr = words + row * row_words;
+  const int cw = CH / 32 * bits, pw = N * bits;  // words of a chunk, bits of a piece
+  T v[N], sv[N], pv[N];
+  auto load = [&](int64_t j) {
+    if (j >= n) return;
+    load_values<T, N>(v, zr, j, n);
+    f.load(sv, pv, j, n);
+  };
+  int nbad = 0, buf = 0;
+  int64_t j = N * t;
+  load(j);
+  for (int64_t w0 = 0; w0 < row_words; w0 += cw, j += CH, buf ^= 1) {
+    uint64_t u = 0;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      if (j + k < n) {
+        bool ok;
+        u |= (uint64_t)int_code(v[k], sv[k], pv[k], qmin, qmax, ok) << (k * bits);
+        nbad += ok ? 0 : 1;
+      }
+    }
+    uint64_t* const mine = pieces[buf][threadIdx.x / TPR];
+    mine[t] = u;
+    load(j + CH);
+    sync();  // one a chunk: the next chunk's pieces go to the other buffer
+    for (int w = t; w < cw && w0 + w < row_words; w += TPR) {
+      // the pieces that overlap the word, the first from its bit `skip` on
+      int k = 32 * w / pw;
+      const int skip = 32 * w - k * pw;
+      uint32_t word = (uint32_t)(mine[k++] >> skip);
+      for (int pos = pw - skip; pos < 32; pos += pw) word |= (uint32_t)mine[k++] << pos;
+      if (live) wr[w0 + w] = word;
+    }
+  }
+  nbad = row_sum<TPR>(nbad, sums);
+  if (t == 0 && live && bad) bad[row] = nbad;
+}
+
+// 4 and 8 bits with one scale and zero point per row: a thread packs the 32 / BITS codes of a word, without LDS.
+// 4096^2 at 4 bits 17.6 us, 8 bits 17.9; the kernel above 21.8 and 22.9.
+template <typename T, int BITS, int TPR>
+__global__ __launch_bounds__(256) void int_pack_words_kernel(const T* __restrict__ z, int64_t rows, int64_t m,
+                                                             int64_t n, IntLayout<T> lay, T qmin, T qmax,
+                                                             uint32_t* __restrict__ words, int64_t row_words,
+                                                             int32_t* __restrict__ bad) {
+  constexpr int N = 32 / BITS;
+  __shared__ int sums[4];
   const int t = threadIdx.x % TPR;
   const int64_t row = (int64_t)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
   if (TPR == 64 && row >= rows) return;  // uniform over the wave
-  const int64_t b = rows == m ? 0 : row / m, i = rows == m ? row : row % m;
+  const IntRow<T> f(lay, row, rows, m, n);
   const T* zr = z + row * n;
-  const T* sr = lay.s + b * lay.sb + i * lay.sm;
-  const T* pr = lay.zp ? lay.zp + b * lay.zb + i * lay.zm : nullptr;
   uint32_t* wr = words + row * row_words;
-  const T s0 = lay.sn ? T(0) : *sr, p0 = pr && !lay.zn ? *pr : T(0);
-  const int wpu = BITS ? 1 : bits;  // words of a unit
   int nbad = 0;
-  for (int64_t unit = t; unit * wpu < row_words; unit += TPR) {
-    const int64_t j = unit * N;
-    uint64_t acc = 0;
+  for (int64_t w = t; w < row_words; w += TPR) {
+    const int64_t j = w * N;
+    uint32_t word = 0;
     if (j < n) {
       T v[N];
       load_values<T, N>(v, zr, j, n);
-      int nacc = 0;
-      int64_t w = unit * wpu;
 #pragma unroll
       for (int k = 0; k < N; ++k) {
         if (j + k < n) {
           bool ok;
-          const uint64_t u = int_code(v[k], lay.sn ? sr[(j + k) * lay.sn] : s0, pr && lay.zn ? pr[(j + k) * lay.zn] : p0,
-                                      qmin, qmax, ok);
+          word |= int_code(v[k], f.s0, f.p0, qmin, qmax, ok) << (k * BITS);
           nbad += ok ? 0 : 1;
-          acc |= u << (BITS ? k * BITS : nacc);
-        }
-        if constexpr (!BITS) {
-          nacc += bits;
-          if (nacc >= 32) {
-            if (w < row_words) wr[w] = (uint32_t)acc;
-            ++w;
-            acc >>= 32;
-            nacc -= 32;
-          }
         }
       }
-      if constexpr (BITS != 0) wr[w] = (uint32_t)acc;
-    } else {
-      for (int64_t w = unit * wpu; w < (unit + 1) * wpu && w < row_words; ++w) wr[w] = 0u;
     }
+    wr[w] = word;
   }
-  nbad = wave_sum(nbad);
-  if constexpr (TPR == 256) {
-    if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = nbad;
-    __syncthreads();
-    nbad = sums[0] + sums[1] + sums[2] + sums[3];
-  }
+  nbad = row_sum<TPR>(nbad, sums);
   if (t == 0 && bad) bad[row] = nbad;
 }
 
-// A thread writes eight consecutive values of a row (gpr groups of eight per row).
+// A thread writes N consecutive values of a row (gpr groups of N per row).  BITS 4 or 8: N = 8 and one scale and zero
+// point per row (fp32; 4096^2 at 4 bits 15.9 us, 20.5 with 16 bytes a thread); BITS 0: any width, N values of 16 bytes
+// (5 bits: one scale per row 21 us, a scale per entry 23, with zero points 32; 8 values a thread 26, 50 and 74).
 template <typename T, int BITS>
 __global__ __launch_bounds__(256) void int_unpack_kernel(const uint32_t* __restrict__ words, int64_t rows, int64_t m,
                                                          int64_t n, int64_t gpr, int64_t row_words, IntLayout<T> lay,
                                                          T qmin, int bits, T* __restrict__ z) {
-  constexpr int N = 8, VE = 16 / (int)sizeof(T);
+  constexpr int VE = 16 / (int)sizeof(T), N = BITS ? 8 : VE;
   typedef T vec_t __attribute__((ext_vector_type(VE), aligned(sizeof(T))));
   const uint32_t mask = (1u << bits) - 1u;
   const int64_t total = rows * gpr;
@@ -151,34 +235,37 @@ __global__ __launch_bounds__(256) void int_unpack_kernel(const uint32_t* __restr
   for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * 256) {
     const int64_t row = small ? (int64_t)((uint32_t)idx / (uint32_t)gpr) : idx / gpr;
     const int64_t j = (idx - row * gpr) * N;
-    const int64_t b = rows == m ? 0 : row / m, i = rows == m ? row : row % m;
     const uint32_t* wr = words + row * row_words;
-    const T* sr = lay.s + b * lay.sb + i * lay.sm;
-    const T* pr = lay.zp ? lay.zp + b * lay.zb + i * lay.zm : nullptr;
-    const T s0 = lay.sn ? T(0) : *sr, p0 = pr && !lay.zn ? *pr : T(0);
-    uint32_t word[2];
-    if constexpr (BITS == 4) word[0] = wr[j >> 3];
-    if constexpr (BITS == 8) {
-      word[0] = wr[j >> 2];
-      word[1] = j + 4 < n ? wr[(j >> 2) + 1] : 0u;
+    // BITS 0: the N codes' bits lie in three words at most (N bits <= 64, from bit `off` of the first)
+    uint32_t word[3] = {0u, 0u, 0u};
+    int off = 0;
+    if constexpr (BITS != 0) {
+      const int64_t w = j * BITS >> 5;
+      word[0] = wr[w];
+      if (BITS == 8 && j + 4 < n) word[1] = wr[w + 1];
+    } else {
+      const int64_t start = j * bits, w = start >> 5;
+      off = (int)(start & 31);
+#pragma unroll
+      for (int x = 0; x < 3; ++x)
+        if ((x == 0 || off + N * bits > 32 * x) && w + x < row_words) word[x] = wr[w + x];
     }
-    T v[N];
+    const IntRow<T> f(lay, row, rows, m, n);
+    T v[N], sv[N], pv[N];
+    if constexpr (BITS == 0) f.load(sv, pv, j, n);
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-      uint32_t u = 0;
+      uint32_t u;
       if constexpr (BITS != 0) {
         u = word[k * BITS / 32] >> (k * BITS % 32);
-      } else if (j + k < n) {
-        const int64_t start = (j + k) * bits, w = start >> 5;
-        const int off = (int)(start & 31);
-        u = wr[w] >> off;
-        if (off + bits > 32) u |= wr[w + 1] << (32 - off);
+        sv[k] = f.s0, pv[k] = f.p0;
+      } else {
+        const int pos = off + k * bits;
+        const uint32_t lo = pos < 32 ? word[0] : (pos < 64 ? word[1] : word[2]), hi = pos < 32 ? word[1] : word[2];
+        u = (uint32_t)((((uint64_t)hi << 32) | lo) >> (pos & 31));
       }
       const T q = T(u & mask) + qmin;
-      const bool in = j + k < n;
-      const T s = lay.sn ? (in ? sr[(j + k) * lay.sn] : T(0)) : s0;
-      const T zp = pr && lay.zn ? (in ? pr[(j + k) * lay.zn] : T(0)) : p0;
-      v[k] = (q - zp) * s;
+      v[k] = (q - pv[k]) * sv[k];
     }
     T* zr = z + row * n + j;
     if (j + N <= n) {
@@ -350,17 +437,30 @@ int pack_int(const T* z, int64_t B, int64_t m, int64_t n, const T* s, const int6
   const int64_t rows = B * m;
   if (rows == 0) return 0;
   if (!int_layout(lay, s, ss, zp, zs)) return GPTQ2D_EINVAL;
-  // a workgroup per row from 256 words on, a wave below (a row too short to feed four waves)
-  auto go = [&](auto kernel, int rows_per_wg) {
+  // 4 and 8 bits, one scale and zero point per row, 256 columns and more (16384 x 256 at 8 bits 7.7 us against 9.5 with
+  // the other kernel, 65536 x 64 at 4 bits 30 against 8): a workgroup per row from 256 words on, a wave below (a row too
+  // short to feed four waves).  Otherwise threads by the row's length, fp32, one scale per row, 3 bits: 65536 x 100 in 14
+  // us by 8 threads and 29 by a wave, 16384 x 256 11 and 9, 2048 x 2048 by a wave 11 and by a workgroup 9, 4096 x 1000 by
+  // a wave 9.  A grid has fewer than 2^32 threads.
+  const bool fixed = lay.sn == 0 && lay.zn == 0 && n >= 256, wide = rows < ((int64_t)1 << 24);
+  auto words_of = [&](auto kernel, int rows_per_wg) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)cdiv(rows, rows_per_wg)), dim3(256), 0, stream, z, rows, m, n, lay, (T)qmin,
+                       (T)qmax, words, row_words, bad);
+  };
+  auto any_width = [&](auto kernel, int rows_per_wg) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)cdiv(rows, rows_per_wg)), dim3(256), 0, stream, z, rows, m, n, lay, (T)qmin,
                        (T)qmax, bits, words, row_words, bad);
   };
-  if (bits == 4)
-    row_words >= 256 ? go(int_pack_kernel<T, 4, 256>, 1) : go(int_pack_kernel<T, 4, 64>, 4);
-  else if (bits == 8)
-    row_words >= 256 ? go(int_pack_kernel<T, 8, 256>, 1) : go(int_pack_kernel<T, 8, 64>, 4);
+  if (fixed && bits == 4)
+    row_words >= 256 && wide ? words_of(int_pack_words_kernel<T, 4, 256>, 1) : words_of(int_pack_words_kernel<T, 4, 64>, 4);
+  else if (fixed && bits == 8)
+    row_words >= 256 && wide ? words_of(int_pack_words_kernel<T, 8, 256>, 1) : words_of(int_pack_words_kernel<T, 8, 64>, 4);
+  else if (n <= 128)
+    any_width(int_pack_kernel<T, 8>, 32);
+  else if (n < 2048 || !wide)
+    any_width(int_pack_kernel<T, 64>, 4);
   else
-    row_words >= 256 * bits ? go(int_pack_kernel<T, 0, 256>, 1) : go(int_pack_kernel<T, 0, 64>, 4);
+    any_width(int_pack_kernel<T, 256>, 1);
   return (int)hipGetLastError();
 }
 
@@ -373,14 +473,16 @@ int unpack_int(const uint32_t* words, int64_t B, int64_t m, int64_t n, int64_t r
   const int64_t total = B * m * n;
   if (total == 0) return 0;
   if (!int_layout(lay, s, ss, zp, zs)) return GPTQ2D_EINVAL;
-  const int64_t gpr = cdiv(n, 8);
+  const bool fixed = sizeof(T) == 4 && lay.sn == 0 && lay.zn == 0;
+  const int group = fixed && (bits == 4 || bits == 8) ? 8 : 16 / (int)sizeof(T);
+  const int64_t gpr = cdiv(n, group);
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(grid_for(B * m * gpr)), dim3(256), 0, stream, words, B * m, m, n, gpr, row_words, lay,
                        (T)qmin, bits, z);
   };
-  if (bits == 4)
+  if (fixed && bits == 4)
     go(int_unpack_kernel<T, 4>);
-  else if (bits == 8)
+  else if (fixed && bits == 8)
     go(int_unpack_kernel<T, 8>);
   else
     go(int_unpack_kernel<T, 0>);
