@@ -822,14 +822,16 @@ int64_t split_bytes(int64_t m, int64_t n, int64_t B, int64_t bl, int64_t bu, Spl
   return 2 * B * ec + bl * lt + bu * ut + B * 4 * (int64_t)sizeof(int64_t);
 }
 
+// Workgroups of split_factors_kernel.
+int64_t factor_groups(int64_t mt, int64_t nt) { return cdiv(mt * (mt - 1) / 2 + nt * (nt - 1) / 2, 2); }
+
 template <bool KR>
 int run(Args& a, int64_t bl, int64_t bu, bool rows, int64_t outer_tiles, int64_t stage_begin, int64_t stage_end) {
   const Split& sp = a.g.sp;
   const int64_t mt = sp.mt, nt = sp.nt, stages = mt + nt - 1;
   int rc;
   if (stage_begin == 0 && (rc = gptq2d_fill<float>(a.g.c, 0.f, a.B * a.m * a.n, a.stream))) return rc;
-  const int64_t nl = mt * (mt - 1) / 2, nu = nt * (nt - 1) / 2, groups = cdiv(nl + nu, 2);
-  if (groups > 0x7fffffff || a.B > 65535) return GPTQ2D_EUNSUPPORTED;
+  const int64_t nl = mt * (mt - 1) / 2, nu = nt * (nt - 1) / 2, groups = factor_groups(mt, nt);
   if (a.g.offsets)
     hipLaunchKernelGGL(batch_offsets_kernel, dim3((unsigned)cdiv(a.B, 256)), dim3(256), 0, a.stream, a.offsets, a.B, a.lmap,
                        a.umap, a.smap, a.zmap);
@@ -908,6 +910,8 @@ int gptq2d_sweep_split_f32(float* y, float* c, float* e, const float* l, const f
   }
   a.B = batch_count(bnd, bshape);
   if (a.B == 0) return 0;
+  // the grids: matrices along y, and below 2^32 threads along x for the factors' blocks and C's
+  if (a.B > 65535 || factor_groups(cdiv(m, TR), cdiv(n, TR)) > ((int64_t)1 << 24) - 4097) return GPTQ2D_EUNSUPPORTED;
   const int64_t bl = shared_over_batch(a.lmap) ? 1 : a.B, bu = shared_over_batch(a.umap) ? 1 : a.B;
   if (!work || ((uintptr_t)work & 15) || work_bytes < split_bytes(m, n, a.B, bl, bu, &a.g.sp, (char*)work))
     return GPTQ2D_EINVAL;

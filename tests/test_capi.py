@@ -63,3 +63,26 @@ def test_every_export_is_declared():
     assert len(exported) > 30
     undeclared = sorted(set(exported) - set(declared_symbols()))
     assert not undeclared, undeclared
+
+
+def test_split_sweep_refuses_before_any_device_work():
+    """gptq2d_sweep_split_f32 returns its code for a call its grids cannot number without touching the device (the
+    pointers are never read: a launch or a fill would report another code, or fault)."""
+    if not LIB.exists():
+        pytest.skip("libgptq2d.so is not built (run __graft_entry__.build())")
+    fn = ctypes.CDLL(str(LIB)).gptq2d_sweep_split_f32
+    i64, i32, f64, p = ctypes.c_int64, ctypes.c_int32, ctypes.c_double, ctypes.c_void_p
+    arr = lambda *v: (i64 * max(1, len(v)))(*v)
+    mem = p(1 << 20)
+
+    def call(m, n, batch, up=None, np_=0, nq=0):
+        none = arr(*[0] * len(batch))
+        return fn(mem, mem, mem, mem, None if up else mem, up, up, i64(np_), i64(nq), i64(m), i64(n), i64(1), i64(1),
+                  i32(len(batch)), arr(*batch), none, none, i32(0), None, none, None, none, f64(0), f64(0), i32(0), None,
+                  None, i64(1), i64(0), i64(-1), mem, i64(1 << 62), None)
+
+    unsupported = -2
+    assert call(1, 1, (65536,)) == unsupported
+    assert call(1, 1, (256, 256)) == unsupported
+    assert call(1, 1 << 20, ()) == unsupported
+    assert call(1, (1 << 20) - 32, (), mem, 1, (1 << 20) - 32) == unsupported  # more than 2^32 threads to split U
