@@ -146,7 +146,7 @@ __global__ __launch_bounds__(256) void split_factors_kernel(const float* __restr
 
 // One wave's share of a band product: acc += sum over the 16-deep halves ch = c_lo + part (mod nparts) below c_hi of
 // the row of left blocks at `a` times the column of right blocks at `b`, straight from global memory.  The loads of G
-// halves are issued before their products; past c_hi the last half is read again and not multiplied.
+// halves are issued before their products.
 template <int G>
 __device__ __forceinline__ void pull_split(floatx16& acc, const char* __restrict__ a, const char* __restrict__ b,
                                            int c_lo, int c_hi, int part, int nparts, int lane) {
@@ -154,9 +154,10 @@ __device__ __forceinline__ void pull_split(floatx16& acc, const char* __restrict
     bf16x8 av[G][3], bv[G][3];
 #pragma unroll
     for (int q = 0; q < G; ++q) {
-      const int ch = base + nparts * q, at = ch < c_hi ? ch : c_hi - 1;
-      const char* ap = a + at * HB + 16 * lane;
-      const char* bp = b + at * HB + 16 * lane;
+      const int ch = base + nparts * q;
+      if (ch >= c_hi) break;
+      const char* ap = a + ch * HB + 16 * lane;
+      const char* bp = b + ch * HB + 16 * lane;
 #pragma unroll
       for (int p = 0; p < 3; ++p) {
         av[q][p] = *reinterpret_cast<const bf16x8*>(ap + 1024 * p);
@@ -216,16 +217,19 @@ __device__ __forceinline__ void pull_exact(floatx16& acc, bool down, const float
 }
 
 // The split E and C of a swept tile of 1 x 32 rows, from its LDS image: threads 0-127 the 128 (half, lane) groups of
-// E's block (column l % 32, rows 16 half + 8 (l / 32) ..), threads 128-255 those of C's (row l % 32, columns ..).
+// E's block (column l % 32, rows 16 half + 8 (l / 32) ..), threads 128-255 those of C's (row l % 32, columns ..).  A block
+// that is null is not written.
 __device__ __forceinline__ void store_split(const TileLds& tl, char* eblk, char* cblk, int rows_in, int cols_in) {
   const int lane = threadIdx.x & 63, half = (threadIdx.x >> 6) & 1;
   const int li = lane & 31, kk = 16 * half + 8 * (lane >> 5);
   float v[8];
   if (threadIdx.x < 128) {
+    if (!eblk) return;
 #pragma unroll
     for (int s = 0; s < 8; ++s) v[s] = kk + s < rows_in && li < cols_in ? tl.Es[TR + kk + s][li] : 0.f;
     store_half(eblk + half * HB, lane, v);
   } else {
+    if (!cblk) return;
 #pragma unroll
     for (int s = 0; s < 8; ++s) v[s] = li < rows_in && kk + s < cols_in ? tl.Cs[li][TR + kk + s] : 0.f;
     store_half(cblk + half * HB, lane, v);
@@ -487,8 +491,14 @@ __global__ __launch_bounds__(NTHREADS, 2) void row_stage_split_kernel(StageArgs 
     const bool down = wave < pr.wd;
     const int c_lo = down ? pr.d0 : pr.r0, c_hi = down ? pr.d1 : pr.r1, part = down ? wave : wave - pr.wd,
               np = down ? pr.wd : 4 - pr.wd;
-    pull_split<4>(acc, down ? sp.l_row(b, I) : sp.c_row(b, I), down ? sp.e_col(b, J) : sp.u_col(b, J), c_lo, c_hi,
-                  part, np, lane);
+    const char* pa = down ? sp.l_row(b, I) : sp.c_row(b, I);
+    const char* pb = down ? sp.e_col(b, J) : sp.u_col(b, J);
+    // a sweep has two halves of a product at most; a prep's path is its loads, and no later launch hides it (1024^2 round
+    // at 512 antidiagonals 702 us with four halves at a time, read again past the last, 592 with six)
+    if (sweep)
+      pull_split<1>(acc, pa, pb, c_lo, c_hi, part, np, lane);
+    else
+      pull_split<6>(acc, pa, pb, c_lo, c_hi, part, np, lane);
     if (any_nonfinite(acc))
       pull_exact<KR>(acc, down, lb, e + mat, c + mat, KR ? nullptr : g.u + off.u, kr, m, n, i0, j0, c_lo, c_hi,
                      part, np, lane);
@@ -516,9 +526,14 @@ __global__ __launch_bounds__(NTHREADS, 2) void row_stage_split_kernel(StageArgs 
   }
   own.store(tl, red, pr.any, pr.wd);
   __syncthreads();
-  sweep_rows<float, KIND, YPRE, true>(&tl.Ys[0][0], SP, &tl.Cs[0][TR], CPW, &tl.Lp[0][TR], LPW, &tl.Es[TR][0], SP, rin,
-                                      y, c, e, qs, m, n, i0, j0, mat);
-  store_split(tl, sp.e_col(b, J) + I * 2 * HB, sp.c_row(b, I) + J * 2 * HB, rows_in, cols_in);
+  // the split blocks that a later tile reads (the last tile row's E and the last tile column's C have none)
+  char* const eblk = I + 1 < sp.mt ? sp.e_col(b, J) + I * 2 * HB : nullptr;
+  char* const cblk = J + 1 < sp.nt ? sp.c_row(b, I) + J * 2 * HB : nullptr;
+  const bool image = eblk || cblk;
+  sweep_rows<float, KIND, YPRE>(&tl.Ys[0][0], SP, &tl.Cs[0][TR], CPW, &tl.Lp[0][TR], LPW, &tl.Es[TR][0], SP, rin, y, c, e,
+                                qs, m, n, i0, j0, mat, image);
+  if (!image) return;
+  store_split(tl, eblk, cblk, rows_in, cols_in);
   store_tile(tl, y, c, e, m, n, i0, j0, mat);
 }
 

@@ -124,16 +124,16 @@ struct RowInputs {
   }
 };
 
-// The TR row steps of one tile, then its Y, C and E to global memory (IMAGE: Y and C to ys and cs instead, beside
-// the published errors in es, and a barrier).  ys / cs: the tile's Y and C with
+// The TR row steps of one tile, then its Y, C and E to global memory (`image`, uniform over the workgroup: Y and C to ys
+// and cs instead, beside the published errors in es, and a barrier).  ys / cs: the tile's Y and C with
 // the pulled feedback (row pitches ysp, csp); lp[r lpp + k] = L[i0 + r, i0 + k] for k < r, zero
 // elsewhere; es: TR x esp floats for the published errors.  Expects the image complete (a barrier after
 // it was written).
-template <typename T, int KIND, bool YPRE, bool IMAGE = false>
+template <typename T, int KIND, bool YPRE>
 __device__ __forceinline__ void sweep_rows(T* ys, int ysp, T* cs, int csp, const T* lp, int lpp, T* es,
                                            int esp, const RowInputs<T, KIND>& in, T* __restrict__ y,
                                            T* __restrict__ c, T* __restrict__ e, const QSpec<T>& qs, int64_t m,
-                                           int64_t n, int64_t i0, int64_t j0, int64_t mat) {
+                                           int64_t n, int64_t i0, int64_t j0, int64_t mat, bool image = false) {
   const int cc = threadIdx.x & 31, g = threadIdx.x >> 5, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rows_in = m - i0 < TR ? (int)(m - i0) : TR;  // the super-entries span the tile's columns
   T Y[4], C[4], D[4], E[4];
@@ -146,7 +146,8 @@ __device__ __forceinline__ void sweep_rows(T* ys, int ysp, T* cs, int csp, const
   const T qmin = qs.qmin, qmax = qs.qmax, half = (qs.qmax - qs.qmin) / T(2);
   auto step = [&](auto r_c) __attribute__((always_inline)) {
     constexpr int r = decltype(r_c)::value, slot = r & 3;
-    if (wave == (r >> 3)) {  // the wave that holds the row; the others wait for its errors
+    // the wave that holds the row; the others wait for its errors (fp64, 512^2 affine: 697 us, 703 with the branch)
+    if (sizeof(T) == 8 || wave == (r >> 3)) {
       const bool own = g == (r >> 2) && r < rows_in;
       const T yv = Y[slot] + D[slot];
       T z, sc = T(1);
@@ -190,7 +191,7 @@ __device__ __forceinline__ void sweep_rows(T* ys, int ysp, T* cs, int csp, const
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = 4 * g + i;
-    if constexpr (IMAGE) {
+    if (image) {
       ys[r * ysp + cc] = Y[i];
       cs[r * csp + cc] = C[i];
     } else if (r < rows_in) {
@@ -200,7 +201,7 @@ __device__ __forceinline__ void sweep_rows(T* ys, int ysp, T* cs, int csp, const
       e[off] = E[i];
     }
   }
-  if constexpr (IMAGE) __syncthreads();
+  if (image) __syncthreads();
 }
 
 // ------------------------------------------------------------------------------------------------ fp32: pull + sweep

@@ -181,3 +181,30 @@ def test_values_that_are_not_finite_elsewhere(form, value, monkeypatch):
     if abs(value) < float("inf"):
         tol[..., at[-2]:, at[-1]:] += (m + n + 4) * 2. ** -23 * value
     assert ((pre - want).abs() <= tol)[ok].all()
+
+
+@pytest.mark.parametrize("m,n,outer", [(1, 32, 64), (32, 32, 64), (31, 64, 64), (96, 32, 512), (130, 96, 32), (257, 640, 512),
+                                       (700, 320, 4096)])
+def test_rows_before_rounding(m, n, outer):
+    """1 x 32 rows: single tiles, the last tile row and column (whose split blocks nobody reads), and preps that pull
+    more halves than are in flight at once (44 of them a product in blocks of 4096 antidiagonals).  The bound of
+    test_values_before_rounding."""
+    print(f"split rows {m}x{n} outer={outer}", flush=True)
+    x, lo, up = _layer(m, n, m + 5 * n)
+    z = torch.round(x)
+
+    def run(dt):
+        pre = torch.full_like(x, torch.nan, dtype=dt)
+        got = G.gptq_2d_super_entry(x.to(dt), lo.to(dt), up.to(dt), super_entry_shape=(1, 32),
+                                    quantizer=QI.teacher_forced_quantizer, quantizer_inputs=(z.to(dt), pre),
+                                    outer_block_size=outer, fused=True)
+        assert got.equal(z.to(dt))
+        return pre.double()
+
+    pre, pre64 = run(torch.float32), run(torch.float64)
+    block = torch.arange(n, device=DEV) // 32
+    l64, u64 = lo.double().tril(-1), torch.where(block[:, None] < block[None], up.double(), 0.)
+    e = z.double() - pre64
+    c = e + l64 @ e
+    size = x.double().abs() + l64.abs() @ e.abs() + c.abs() @ u64.abs() + (l64.abs() @ e.abs()) @ u64.abs()
+    assert ((pre - pre64).abs() <= (m + n + 4) * 2. ** -23 * size).all()
