@@ -173,8 +173,13 @@ def i64_array(values) -> ctypes.Array:
     return (ctypes.c_int64 * max(1, len(values)))(*(values or [0]))
 
 
+_NO_BATCH = i64_array(())
+
+
 def batch_strides(x: torch.Tensor, batch_shape: torch.Size) -> ctypes.Array:
     """Batch strides of matrix-shaped ``x`` broadcast to ``batch_shape`` (0 on broadcast dims)."""
+    if not batch_shape:
+        return _NO_BATCH
     pad = len(batch_shape) - (x.dim() - 2)
     view = x.reshape((1,) * pad + tuple(x.shape)).expand(*batch_shape, *x.shape[-2:])
     return i64_array(view.stride()[:-2])

@@ -225,7 +225,7 @@ def _run_split(y, l, u, m, n, batch_shape, spec, outer_block_size, p, q):
     kron = isinstance(u, KroneckerU)
     bshape, nd = _hip.i64_array(batch_shape), len(batch_shape)
     lstr = _hip.batch_strides(l, batch_shape)
-    ustr = _hip.i64_array([0] * nd) if kron else _hip.batch_strides(u, batch_shape)
+    ustr = lstr if kron else _hip.batch_strides(u, batch_shape)  # a Kronecker U comes without a batch
     need = _hip.lib().gptq2d_sweep_split_workspace(m, n, nd, bshape, lstr, ustr)
     if not 0 <= need <= SPLIT_WORKSPACE_MAX:
         return False
