@@ -38,9 +38,10 @@ def _side_streams(device: torch.device):
 
 
 # Sizes from which, and below which, a matrix whose rows are not on 16-byte boundaries is factored inside an
-# aligned one: 602 fp32 1.15 -> 0.44 ms, 1531 3.20 -> 1.00, 8190 23.5 -> 7.6; fp64 777 0.91 -> 0.70, 4099 5.41 ->
-# 4.04.  Smaller ones keep the library's own sequence, the one its entry points for parts of a factorisation take
-# (301 fp32: 0.48 against 0.29 ms); from PAD_MAX on the two larger copies would be 1 GiB (fp32) and more each.
+# aligned one: fp32 1531 3.20 -> 1.00 ms, 8190 23.5 -> 7.6; fp64 777 0.91 -> 0.70, 4099 5.41 -> 4.04.  Smaller ones
+# would gain as well (fp32 301 0.48 -> 0.29, 602 1.15 -> 0.44), but keep the library's own sequence, the one its
+# entry points for parts of a factorisation take, so that parts and whole agree bit for bit there; from PAD_MAX on the
+# two larger copies would be 1 GiB (fp32) and more each.
 PAD_MIN, PAD_MAX = 640, 16384
 
 
@@ -57,11 +58,24 @@ def _pad(m: torch.Tensor, size: int) -> int:
     return pad
 
 
-def _embed(m: torch.Tensor, kd: int, off: int) -> torch.Tensor:
+def _embed(m: torch.Tensor, kd: int, off: int, out: torch.Tensor | None = None) -> torch.Tensor:
     """[batch, k, k] at row and column off of a kd x kd identity; kd < k: its part from -off on."""
-    out = m.new_empty(m.size(0), kd, kd)
+    out = m.new_empty(m.size(0), kd, kd) if out is None else out
     _hip.call("embed", m.dtype, _hip.ptr(out), _hip.ptr(m), m.size(0), kd, m.size(-1), off, _hip.stream(m.device))
     return out
+
+
+def _buffers(src: torch.Tensor, pad: int, lead: int):
+    """(rows added, matrix, output, work, the factor taken out): src inside a matrix of `pad` more rows, `lead` of them
+    before it, or, where the device has no room for these, as it is."""
+    if pad:
+        try:
+            big = src.new_empty(src.size(0), src.size(-1) + pad, src.size(-1) + pad)
+            more = torch.empty_like(big), torch.empty_like(big), torch.empty_like(src)
+            return pad, _embed(src, big.size(-1), lead, big), *more
+        except torch.OutOfMemoryError:
+            big = None  # given back before the smaller ones are asked for
+    return 0, src, torch.empty_like(src), torch.empty_like(src), None
 
 
 def _factor(name: str, m: torch.Tensor, size: int, check: bool) -> torch.Tensor:
@@ -80,14 +94,11 @@ def _factor(name: str, m: torch.Tensor, size: int, check: bool) -> torch.Tensor:
     # ldl_of_inverse, after it for ldl, so that info counts the minors of M
     lead = pad if name == "ldl_of_inverse" else 0
     with torch.cuda.device(m.device):
-        if pad:
-            src = _embed(src, k + pad, lead)
-        out = torch.empty_like(src)
-        work = torch.empty_like(src)
+        pad, src, out, work, part = _buffers(src, pad, lead)
         _hip.call(name, m.dtype, _hip.ptr(src), _hip.ptr(out), _hip.ptr(work), _hip.ptr(info), nb, k + pad, size,
                   _hip.stream(m.device))
         if pad:
-            out = _embed(out, k, -lead)
+            out = _embed(out, k, -lead, part)
     if check and nb and k:
         bad = info.cpu()
         if bool((bad != 0).any()):
@@ -140,19 +151,19 @@ def feedback_factors_of_grams(G: torch.Tensor, H: torch.Tensor, super_entry_shap
         k = m.size(-1)
         assert size > 0 and k % size == 0, "the block size must divide the matrix size"
         assert size <= MAX_BLOCK[m.dtype], f"diagonal blocks up to {MAX_BLOCK[m.dtype]} are supported for {m.dtype}"
-        jobs.append((m, size, k, _pad(m, size)))
+        jobs.append((m, size, k))
     out = []
     upper = False  # whether out[1] holds U itself (else the second factor, U its transpose)
     with torch.cuda.device(G.device):
         # each factor's buffers on its stream's pool
-        bufs = []
-        for s, (m, size, k, pad) in zip(streams, jobs):
+        bufs, parts = [], []
+        for f, (s, (m, size, k)) in enumerate(zip(streams, jobs)):
             with torch.cuda.stream(s):
-                src = m.reshape(-1, k, k).contiguous()
-                if pad:
-                    src = _embed(src, k + pad, pad)
-                bufs.append((src, torch.empty_like(src), torch.empty_like(src),
-                             torch.zeros(src.size(0), dtype=torch.int32, device=m.device)))
+                pad = _pad(m, size)
+                pad, *buf, part = _buffers(m.reshape(-1, k, k).contiguous(), pad, pad)
+                jobs[f] = (m, size, k, pad)
+                parts.append(part)
+                bufs.append((*buf, torch.zeros(buf[0].size(0), dtype=torch.int32, device=m.device)))
         (sa, oa, wa, ia), (sb, ob, wb, ib) = bufs
         (_, pa, ka, da), (_, pb, kb, db) = jobs
         if max(sa.size(0), sb.size(0)) > 1:
@@ -178,7 +189,7 @@ def feedback_factors_of_grams(G: torch.Tensor, H: torch.Tensor, super_entry_shap
         for f, s in enumerate(streams[:2]):
             if jobs[f][3]:
                 with torch.cuda.stream(s):  # U' = diag(I, U) as L' = diag(I, L)
-                    out.append(_embed((oa, ob)[f], jobs[f][2], -jobs[f][3]))
+                    out.append(_embed((oa, ob)[f], jobs[f][2], -jobs[f][3], parts[f]))
             else:
                 out.append((oa, ob)[f])
         out = [t.reshape(m.shape) for t, m in zip(out, (G, H))]

@@ -103,3 +103,31 @@ def test_padded_under_capture():
         graph.replay()
         torch.cuda.synchronize()
         assert out.equal(LDL.ldl_of_inverse(x))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_no_room_for_the_embedding(dtype, monkeypatch):
+    """Where the allocator refuses what the embedding takes, the matrix is factored as it is: equal bit for bit to the
+    factorisation without an embedding, alone, in a pair and in a batch."""
+    k, kb = 1027, 1030
+    m = torch.stack([instances.wishart_factor(k, .5, s) for s in (1, 2)]).to(DEV, dtype)
+    h = torch.stack([instances.wishart_factor(kb, .5, s) for s in (3, 4)]).to(DEV, dtype)
+    cat = lambda pair: torch.cat([t.flatten() for t in pair])
+    calls = (lambda: LDL.ldl_of_inverse(m[0]), lambda: LDL.ldl(m[0]), lambda: LDL.ldl_of_inverse(m),
+             lambda: cat(LDL.feedback_factors_of_grams(m[0], h[0])), lambda: cat(LDL.feedback_factors_of_grams(m, h)))
+    with monkeypatch.context() as mp:
+        mp.setattr(LDL, "PAD_MIN", LDL.PAD_MAX)
+        want = [f() for f in calls]
+    empty_like, refused = torch.empty_like, []
+
+    def refuse(t):
+        if t.size(-1) not in (k, kb):
+            refused.append(t.shape)
+            raise torch.OutOfMemoryError("no room")
+        return empty_like(t)
+
+    monkeypatch.setattr(torch, "empty_like", refuse)
+    for i, (f, w) in enumerate(zip(calls, want)):
+        print(f"no room for the embedding: call {i}, {dtype}", flush=True)
+        assert f().equal(w)
+    assert len(refused) == (7 if dtype == torch.float32 else 5)  # fp64: rows of 1030 are on 16-byte boundaries
