@@ -41,16 +41,22 @@ def _side_streams(device: torch.device):
 # aligned one: fp32 1531 3.20 -> 1.00 ms, 8190 23.5 -> 7.6; fp64 777 0.91 -> 0.70, 4099 5.41 -> 4.04.  Smaller ones
 # would gain as well (fp32 301 0.48 -> 0.29, 602 1.15 -> 0.44), but keep the library's own sequence, the one its
 # entry points for parts of a factorisation take, so that parts and whole agree bit for bit there; from PAD_MAX on the
-# two larger copies would be 1 GiB (fp32) and more each.
+# two larger copies would be 1 GiB (fp32) and more each.  fp32 ldl stays as it is from LDL_F32_MAX on: its own
+# sequence rounds the trailing entries less often than the two-level one (relative error against 64 bits at 777
+# 6.3e-8 against 5.9e-8 embedded, at 901 6.19e-8 against 6.23e-8, at 1531 5.95e-8 against 6.69e-8, at 3003 4.85e-8 against
+# 5.65e-8).  The inverse's products outweigh that: ldl_of_inverse 1.31e-7 against 1.18e-7 at 901, 1.85e-7 against 1.61e-7
+# at 3003; in fp64 the errors agree to three digits.
 PAD_MIN, PAD_MAX = 640, 16384
+LDL_F32_MAX = 832
 
 
-def _pad(m: torch.Tensor, size: int) -> int:
+def _pad(m: torch.Tensor, size: int, name: str = "ldl_of_inverse") -> int:
     """Rows of identity to add to m (a multiple of the block size) so that the kernels that move 16 bytes of a
     row at a time take it: fp32 the two-level factorisation and the MFMA inverse levels, fp64 the strip's
     narrow product.  (A batch the embedding's grid cannot number stays as it is.)"""
     k, align = m.size(-1), 16 // m.element_size()
-    if k % align == 0 or not PAD_MIN <= k < PAD_MAX or m.numel() > 65535 * k * k:
+    hi = LDL_F32_MAX if name == "ldl" and m.dtype == torch.float32 else PAD_MAX
+    if k % align == 0 or not PAD_MIN <= k < hi or m.numel() > 65535 * k * k:
         return 0
     pad = size
     while (k + pad) % align:
@@ -89,7 +95,7 @@ def _factor(name: str, m: torch.Tensor, size: int, check: bool) -> torch.Tensor:
     src = m.reshape(-1, k, k).contiguous()
     nb = src.size(0)
     info = torch.zeros(nb, dtype=torch.int32, device=m.device)
-    pad = _pad(src, size)
+    pad = _pad(src, size, name)
     # the identity goes where the factorisation comes last: before M for the reversed order of
     # ldl_of_inverse, after it for ldl, so that info counts the minors of M
     lead = pad if name == "ldl_of_inverse" else 0
