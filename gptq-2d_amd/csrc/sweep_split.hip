@@ -3,14 +3,13 @@
 // The schedule is that of sweep_tiles.hip: 32 x 32 tiles by coarse stages T = I + J, one launch per stage (the
 // stage's tiles are swept in LDS while other workgroups pull the next stage's in-block feedback), and after each
 // outer block one flush of its errors into all later stages.  What differs is how a product of two fp32 matrices
-// is formed.  Each operand is held as three bf16 pieces, x = h + m + l with h = bf16(x), m = bf16(x - h), l =
-// bf16(x - h - m) (24 bits together: exact but for pieces below 2^-133), and a product takes the six piece
-// products of weight 2^-16 and above, each exact, on v_mfma_f32_32x32x16_bf16 with fp32 accumulation:
-//   x y = hh' + hm' + mh' + mm' + hl' + lh'   (left out: ml', lm', ll', below 2^-25 |x y| each).
-// Against 64 bits the sums are closer than v_mfma_f32_32x32x2_f32's, whose every two terms round the
-// accumulator (one wave's 32 x 32 block, normal operands: K = 32 6.8e-8 against 1.03e-7 relative, 256 2.4e-7
-// against 2.9e-7, 768 4.2e-7 against 5.0e-7, 4096 1.00e-6 against 1.15e-6), and six bf16 instructions of 32
-// cycles replace eight fp32 ones of 64 (measured peaks on an MI355X: 1865 / 6 = 311 against 135 TFLOP/s).
+// is formed.  Each operand is held as three bf16 pieces, x = h + m + l (split_mma.h: h rounded to nearest, m truncated; 24
+// bits together: exact but for pieces below 2^-133), and a product takes the six piece products of weight 2^-16 and
+// above, each exact, on v_mfma_f32_32x32x16_bf16 with fp32 accumulation:
+//   x y = hh' + hm' + mh' + mm' + hl' + lh'   (left out: ml', lm', below 2^-24 |x y| each, and ll', below 2^-32).
+// Against 64 bits the sums are closer than v_mfma_f32_32x32x2_f32's, whose every two terms round the accumulator (the
+// figures are in split_mma.h), and six bf16 instructions of 32 cycles replace eight fp32 ones of 64 (measured peaks on
+// an MI355X: 1865 / 6 = 311 against 135 TFLOP/s).
 //
 // Split operands are stored as the instruction reads them, one 6 KB block per 32 x 32 tile in two 16-deep halves
 // of three 1 KB pieces: [half][piece][lane][8], lane l holding k = 16 half + 8 (l / 32) + 0..7 of row (left
@@ -152,8 +151,10 @@ __global__ __launch_bounds__(256) void split_factors_kernel(const float* __restr
 
 // One wave's share of a band product: acc += sum over the 16-deep halves ch = c_lo + part (mod nparts) below c_hi of
 // the row of left blocks at `a` times the column of right blocks at `b`, straight from global memory.  The loads of G
-// halves are issued before their products.
-template <int G>
+// halves are issued before their products; FULL: G of them always, the last half again past c_hi (not multiplied), so
+// that no branch lies between them.  FULL suits the plain tiles' two halves at a time (4096^2 at 512 antidiagonals 4.371 ms,
+// 4.395 without; at 768 it is the other way, 3000^2 2.89, 2.82), not the rows' six.
+template <int G, bool FULL>
 __device__ __forceinline__ void pull_split(floatx16& acc, const char* __restrict__ a, const char* __restrict__ b,
                                            int c_lo, int c_hi, int part, int nparts, int lane) {
   for (int base = c_lo + part; base < c_hi; base += nparts * G) {
@@ -161,9 +162,10 @@ __device__ __forceinline__ void pull_split(floatx16& acc, const char* __restrict
 #pragma unroll
     for (int q = 0; q < G; ++q) {
       const int ch = base + nparts * q;
-      if (ch >= c_hi) break;
-      const char* ap = a + ch * HB + 16 * lane;
-      const char* bp = b + ch * HB + 16 * lane;
+      if (!FULL && ch >= c_hi) break;
+      const int at = ch < c_hi ? ch : c_hi - 1;
+      const char* ap = a + at * HB + 16 * lane;
+      const char* bp = b + at * HB + 16 * lane;
 #pragma unroll
       for (int p = 0; p < 3; ++p) {
         av[q][p] = *reinterpret_cast<const bf16x8*>(ap + 1024 * p);
@@ -300,7 +302,7 @@ __global__ __launch_bounds__(DTHREADS, 2) void tile_stage_split_kernel(StageArgs
   const int rows_in = m - i0 < TR ? m - i0 : TR, cols_in = n - j0 < TR ? n - j0 : TR;
 
   if (!sweep) {  // Y += D + R, C += D in place
-    pull_split<2>(acc, pa, pb, c_lo, c_hi, part, np, lane);
+    pull_split<2, true>(acc, pa, pb, c_lo, c_hi, part, np, lane);
     stash();
     __syncthreads();
 #pragma unroll
@@ -502,9 +504,9 @@ __global__ __launch_bounds__(NTHREADS, 2) void row_stage_split_kernel(StageArgs 
     // a sweep has two halves of a product at most; a prep's path is its loads, and no later launch hides it (1024^2 round
     // at 512 antidiagonals 702 us with four halves at a time, read again past the last, 592 with six)
     if (sweep)
-      pull_split<1>(acc, pa, pb, c_lo, c_hi, part, np, lane);
+      pull_split<1, false>(acc, pa, pb, c_lo, c_hi, part, np, lane);
     else
-      pull_split<6>(acc, pa, pb, c_lo, c_hi, part, np, lane);
+      pull_split<6, false>(acc, pa, pb, c_lo, c_hi, part, np, lane);
     if (any_nonfinite(acc))
       pull_exact<KR>(acc, down, lb, e + mat, c + mat, KR ? nullptr : g.u + off.u, kr, m, n, i0, j0, c_lo, c_hi,
                      part, np, lane);
