@@ -21,7 +21,7 @@ LIB = HERE / "libgptq2d.so"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-# -packed-fp32-ops: no v_pk_{add,mul,fma}_f32, which are not trusted on these boxes.
+# -packed-fp32-ops: no v_pk_{add,mul,fma}_f32, some forms of which have given wrong results on this hardware.
 COMMON_FLAGS = [
     f"--offload-arch={ARCH}",
     "-O3",

@@ -1,7 +1,10 @@
 // fp32 products on the bf16 matrix cores: every operand split into three bf16 pieces, x = h + m + l, and six of the
-// nine piece products summed in fp32 (the three left out are below 2^-26 of the product).  6 v_mfma_f32_32x32x16_bf16
-// replace 8 v_mfma_f32_32x32x2_f32 of twice the cycles each, with a smaller error than those (K = 768: 4.2e-7 of the
-// largest entry against 5.0e-7).
+// nine piece products summed in fp32.  What is left out of x y, m l' + l m' + l l', is below 2^-22.9 of it (2^-23.03 for
+// both at 1 + 2^-8 - 2^-23) and 2^-26.0 in the root mean square of normal operands, a quarter of an fp32 rounding's.
+// 6 v_mfma_f32_32x32x16_bf16 replace 8 v_mfma_f32_32x32x2_f32 of twice the cycles each, which round the accumulator
+// every two terms: the sums are closer to 64 bits than theirs.  Relative error in norm: factors of 1024 1.36e-7 on the
+// fp32 MFMA, 1.20e-7 here, 8192 2.33e-7, 1.87e-7; the feedback of a forced sweep of 256^2 8.7e-7, 7.5e-7, 3000 x 4095
+// 1.388e-6, 1.295e-6.
 #pragma once
 
 #include "common.h"
@@ -14,9 +17,11 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 
-// x = h + m + l in bf16 pieces, eight values at once: h rounded to nearest (so that m has no sign of its own and the
-// products left out cancel), m the leading eight bits of the rest, l the last eight.  Whole-register integer steps and
-// byte permutes, 6.5 instructions a value; the conversions to bf16 take 7.5.
+// x = h + m + l in bf16 pieces, exactly, eight values at once: h rounded to nearest, m the leading eight bits of the rest,
+// l the last eight.  m and l have one sign, which for two different operands is random, so that the products left out
+// cancel in a sum; a sum of squares (the diagonal of P P^T) lacks 2^-26.1 of itself.  Whole-register integer steps and
+// byte permutes, 6.5 instructions a value.  m rounded to nearest takes 7.5 (at most 2^-24.2 left out, 2^-27.4 rms, no bias
+// in squares): factors of 1000 to 3072 1.0-1.6 % slower for 1-3 % less error, the sweep's error the same to three digits.
 __device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&p)[3]) {
   typedef unsigned uint4v __attribute__((ext_vector_type(4)));
   uint4v w[3];
