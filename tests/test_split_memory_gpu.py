@@ -3,6 +3,7 @@ batch, a Kronecker U and 1 x 32 rows, against the fp64 sweep under the same code
 limit holds C and E but not the pieces."""
 
 import functools
+import gc
 
 import pytest
 import torch
@@ -96,10 +97,18 @@ def test_allocator_limit():
     pre = torch.empty_like(x)
     _forced(G.gptq_2d, x, lo, up, want, pre_want)
     torch.cuda.synchronize()
+    gc.collect()
     torch.cuda.empty_cache()
-    total = torch.cuda.mem_get_info()[1]
-    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (256 << 20)) / total)
+    total, hold, size = torch.cuda.mem_get_info()[1], [], 1 << 30
     try:
+        # what other tensors' segments have free, so that only the room left below counts
+        torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / total)
+        while size >= 1 << 20:
+            try:
+                hold.append(torch.empty(size, dtype=torch.uint8, device=DEV))
+            except torch.OutOfMemoryError:
+                size >>= 1
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (256 << 20)) / total)
         with pytest.raises(torch.OutOfMemoryError):
             torch.empty(480 << 20, dtype=torch.uint8, device=DEV)
         _forced(G.gptq_2d, x, lo, up, want, pre)

@@ -34,7 +34,7 @@ SIZES = [(1, 1), (1, 40), (33, 1), (31, 33), (32, 32), (64, 65), (95, 129), (257
 @pytest.mark.parametrize("outer", [32, 96, 512])
 def test_values_before_rounding(m, n, outer):
     """Each fp32 sum of up to m + n products errs by at most (m + n + 4) 2^-23 times the sum of the products' magnitudes
-    (every piece product left out is below 2^-23.9 of its product, the three together below 2^-23)."""
+    (the piece products left out are below 2^-22.9 of their product together)."""
     print(f"split sweep {m}x{n} outer={outer}", flush=True)
     x, lo, up = _layer(m, n, m + 3 * n)
     z = torch.round(x)
