@@ -502,7 +502,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void row_stage_split_kernel(StageArgs 
     const char* pa = down ? sp.l_row(b, I) : sp.c_row(b, I);
     const char* pb = down ? sp.e_col(b, J) : sp.u_col(b, J);
     // a sweep has two halves of a product at most; a prep's path is its loads, and no later launch hides it (1024^2 round
-    // at 512 antidiagonals 702 us with four halves at a time, read again past the last, 592 with six)
+    // at 512 antidiagonals 702 us with four halves at a time, read again past the last, 604 with six)
     if (sweep)
       pull_split<1, false>(acc, pa, pb, c_lo, c_hi, part, np, lane);
     else
